@@ -31,6 +31,11 @@ constexpr int kTailBlocksPerCu = 5;
 constexpr int kTailWideOneBlocksPerCu = 6;
 constexpr int kTailFlatBlocksPerCu = 8;
 constexpr uint32_t kSortMinNodes = 1u << 21;
+// render bounces by the group walk from this many primitives on (wavefront
+// renders of 5.2 M paths, lane walk -> group walk: 488 spheres 3.1 -> 3.5 ms,
+// 1000 primitives 2.2 -> 2.5, 50 k 7.1 -> 6.4, 190 k 10.4 -> 9.2, 800 k
+// overlapping 10.0 -> 7.4)
+constexpr uint32_t kGroupMinPrims = 16384;
 
 struct aurora_ctx {
     int device = 0;
@@ -82,19 +87,19 @@ struct aurora_scene {
 // hipGetSymbolAddress (scratch_address, called by aurora_create) and kept
 // in the context.
 constexpr uint32_t kNoAllocMaxRays = AURORA_NOALLOC_MAX_RAYS;
-constexpr int kNoAllocGrid = 512;  // two 256-thread blocks per CU
+constexpr int kNoAllocGrid = 511;  // about two 256-thread blocks per CU
 constexpr size_t kNaRayBytes = (size_t)kNoAllocMaxRays * 16;  // float4 per ray, origins then directions
 constexpr size_t kNaHitBytes = (size_t)kNoAllocMaxRays * 8;   // float2 (t, prim) per ray
 constexpr size_t kNaPoolBytes = (size_t)kPools * kPoolStride * 4;
 constexpr size_t kNaRecBytes = 1024;
-constexpr size_t kNaSpillBytes = (size_t)kNoAllocGrid * kExtendBlock * kExtendSpillLevels * 4;
+constexpr size_t kNaSpillBytes = (size_t)kNoAllocGrid * kExtendBlock * 80 * 4;
 constexpr size_t kNaOffDir = kNaRayBytes;
 constexpr size_t kNaOffHit = 2 * kNaRayBytes;
 constexpr size_t kNaOffPool = kNaOffHit + kNaHitBytes;
 constexpr size_t kNaOffRec = kNaOffPool + kNaPoolBytes;
 constexpr size_t kNaOffSpill = kNaOffRec + kNaRecBytes;
-constexpr size_t kNoAllocScratchBytes = kNaOffSpill + kNaSpillBytes;
-static_assert(kNoAllocScratchBytes == AURORA_NOALLOC_SCRATCH_BYTES, "scratch size stated in aurora.h");
+constexpr size_t kNoAllocScratchBytes = AURORA_NOALLOC_SCRATCH_BYTES;
+static_assert(kNaOffSpill + kNaSpillBytes <= kNoAllocScratchBytes, "scratch size stated in aurora.h");
 static_assert(sizeof(SceneRec) <= kNaRecBytes, "scene record fits its slot");
 static_assert(kNaOffDir % 256 == 0 && kNaOffHit % 256 == 0 && kNaOffPool % 256 == 0 && kNaOffRec % 256 == 0 &&
                   kNaOffSpill % 256 == 0,
@@ -126,7 +131,7 @@ Status scratch_address(int device, unsigned char** out) {
 // capturable)
 __global__ void k_noalloc_setup(uint32_t* pool, SceneRec* rec, SceneRec value) {
     const uint32_t t = threadIdx.x;
-    if (t < (uint32_t)(kPools * kPoolStride)) pool[t] = 0u;
+    if (t < (uint32_t)kPools) pool[kPoolStride * t] = 0u;
     if (t == 0) *rec = value;
 }
 
@@ -321,8 +326,44 @@ int grid_for_extend(aurora_ctx* c, uint64_t n) {
     return (int)std::max<uint64_t>(1, std::min<uint64_t>(need, (uint64_t)c->ext_grid));
 }
 
+// blocks of a group walk over n rays: 16 rays per wave
+int grid_for_group(aurora_ctx* c, uint64_t n) {
+    const uint64_t need = (n + kGroupBlockRays - 1) / kGroupBlockRays;
+    return (int)std::max<uint64_t>(1, std::min<uint64_t>(need, (uint64_t)c->ext_grid));
+}
+
+GroupScene group_scene(const DevScene& v, float tmin) {
+    GroupScene g{};
+    g.wide = v.wide;
+    g.spheres = v.spheres;
+    g.quads = v.quads;
+    g.n_wide = v.n_wide;
+    g.n_spheres = v.n_spheres;
+    g.n_prims = v.n_spheres + v.n_quads;
+    g.tmin = tmin;
+    return g;
+}
+
 Status ensure_spill(DevBuf& spill, int grid) {
     return spill.alloc((size_t)grid * extend_block() * extend_spill_levels() * 4);
+}
+
+bool overlap(const void* a, size_t na, const void* b, size_t nb) {
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return x < y + nb && y < x + na;
+}
+// hits written over rays of the same call: the query reads copies then
+bool hits_over_rays(const float* o, const float* d, const int32_t* prim, const float* t, uint32_t n) {
+    const size_t r = (size_t)n * 12, h = (size_t)n * 4;
+    return overlap(o, r, prim, h) || overlap(o, r, t, h) || overlap(d, r, prim, h) || overlap(d, r, t, h);
+}
+__global__ void k_copy3(const float* src, float* dst, uint32_t n) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const v3 v = load3(src, i);
+    dst[3 * (size_t)i] = v.x;
+    dst[3 * (size_t)i + 1] = v.y;
+    dst[3 * (size_t)i + 2] = v.z;
 }
 
 Status trace_device(aurora_scene* s, const float* o, const float* d, uint32_t n, float tmin, float tmax,
@@ -331,10 +372,68 @@ Status trace_device(aurora_scene* s, const float* o, const float* d, uint32_t n,
     aurora_ctx* c = s->ctx;
     if (!brute && !s->built) return Status{AURORA_ERR_STATE, "BVH not built: call aurora_bvh_build first"};
     if (n == 0) return Status::ok();
+    const uint32_t blocks = (n + 255) / 256;
+    if (!brute && !counts && !count_fetches) {
+        // no counters: the group walk on the caller's rays and hits
+        const int grid = grid_for_group(c, n);
+        if (hits_over_rays(o, d, prim, t, n)) {
+            AUR_TRY(s->tr_o.alloc((size_t)n * 16));
+            AUR_TRY(s->tr_d.alloc((size_t)n * 16));
+            k_copy3<<<blocks, 256, 0, c->stream>>>(o, s->tr_o.as<float>(), n);
+            k_copy3<<<blocks, 256, 0, c->stream>>>(d, s->tr_d.as<float>(), n);
+            o = s->tr_o.as<float>();
+            d = s->tr_d.as<float>();
+        }
+        QueryArgs q{};
+        q.org = o;
+        q.dir = d;
+        q.n = n;
+        q.sc = group_scene(s->view, tmin);
+        q.tmax = tmax;
+        q.prim = prim;
+        q.t = t;
+        AUR_TRY(ensure_spill(s->tr_spill, grid));
+        q.spill = s->tr_spill.as<uint32_t>();
+        q.spill_stride = (uint32_t)(grid * extend_block());
+        AUR_TRY(s->tr_pool.alloc(kPools * kPoolStride * 4));
+        q.pool = s->tr_pool.as<uint32_t>();
+        const bool sort = s->stats.n_nodes > 0 &&
+                          (c->ray_sort == 2 ||
+                           (c->ray_sort == 1 && n >= kSortMinRays && s->stats.n_nodes >= kSortMinNodes));
+        if (sort) {
+            for (int k = 0; k < 2; ++k) {
+                AUR_TRY(s->tr_key[k].alloc((size_t)n * 4));
+                AUR_TRY(s->tr_val[k].alloc((size_t)n * 4));
+            }
+            AUR_TRY(s->tr_hist.alloc(radix_hist_bytes(n)));
+            q.order = s->tr_val[0].as<uint32_t>();
+        }
+        EventPair ev;
+        if (ts) {
+            AUR_TRY(ev.create());
+            AUR_HIP(hipEventRecord(ev.e[0], c->stream));
+        }
+        if (sort) {
+            AUR_TRY(launch_ray_keys(o, d, n, s->view.nodes, s->tr_key[0].as<uint32_t>(), s->tr_val[0].as<uint32_t>(),
+                                    c->stream));
+            AUR_TRY(radix_sort_pairs(s->tr_key[0].as<uint32_t>(), s->tr_val[0].as<uint32_t>(),
+                                     s->tr_key[1].as<uint32_t>(), s->tr_val[1].as<uint32_t>(),
+                                     s->tr_hist.as<uint32_t>(), n, 4, c->stream));
+        }
+        AUR_TRY(launch_query(q, grid, c->stream));
+        if (ts) {
+            AUR_HIP(hipEventRecord(ev.e[1], c->stream));
+            AUR_HIP(hipEventSynchronize(ev.e[1]));
+            float ms = 0.0f;
+            AUR_HIP(hipEventElapsedTime(&ms, ev.e[0], ev.e[1]));
+            *ts = aurora_trace_stats{};
+            ts->extend_ms = ms;
+        }
+        return Status::ok();
+    }
     AUR_TRY(s->tr_o.alloc((size_t)n * 16));
     AUR_TRY(s->tr_d.alloc((size_t)n * 16));
     AUR_TRY(s->tr_hit.alloc((size_t)n * 8));
-    const uint32_t blocks = (n + 255) / 256;
     k_pack3<<<blocks, 256, 0, c->stream>>>(o, s->tr_o.as<float4>(), n);
     k_pack3<<<blocks, 256, 0, c->stream>>>(d, s->tr_d.as<float4>(), n);
     AUR_HIP(hipGetLastError());
@@ -394,7 +493,7 @@ Status trace_device(aurora_scene* s, const float* o, const float* d, uint32_t n,
         hipEvent_t e0 = ev.e[0], e1 = ev.e[1];
         Status ls;
         if (sort) {
-            ls = launch_ray_keys(a.ray_o, a.ray_d, n, s->view.nodes, s->tr_key[0].as<uint32_t>(),
+            ls = launch_ray_keys(o, d, n, s->view.nodes, s->tr_key[0].as<uint32_t>(),
                                  s->tr_val[0].as<uint32_t>(), c->stream);
             if (!ls.bad())
                 ls = radix_sort_pairs(s->tr_key[0].as<uint32_t>(), s->tr_val[0].as<uint32_t>(),
@@ -540,6 +639,15 @@ Status render_jobs(aurora_ctx* c, std::vector<Job>& jobs, aurora_render_stats* s
     // the passes walk the flat leaf array under the condition render_jobs
     // sets pa.flat by (one scene, small enough to have the array)
     const bool flat = c->render_tree == 2 && jobs.size() == 1 && jobs[0].scene->view.n_flat > 0;
+    // four-wide wavefront bounces: the group walk where most paths are in
+    // scenes of at least kGroupMinPrims primitives, one lane per ray elsewhere
+    uint64_t big = 0, all = 0;
+    for (const Job& j : jobs) {
+        const uint64_t p = (uint64_t)j.cam.W * j.cam.H * j.rd.spp;
+        all += p;
+        big += j.scene->n_prims >= kGroupMinPrims ? p : 0u;
+    }
+    const bool group = c->render_tree != 0 && 2 * big >= all;
     const bool wide_one = !flat && c->render_tree != 0 && jobs.size() == 1;
     const int tail_grid =
         c->cus * (flat ? kTailFlatBlocksPerCu : wide_one ? kTailWideOneBlocksPerCu : kTailBlocksPerCu);
@@ -664,7 +772,8 @@ Status render_jobs(aurora_ctx* c, std::vector<Job>& jobs, aurora_render_stats* s
         a.hit = w.hit.as<float2>();
         a.recs = w.recs.as<SceneRec>();
         a.one_scene = jobs.size() == 1;
-        a.wide = c->render_tree != 0 ? 1u : 0u;  // the counting runs trace as the timed ones do
+        a.wide = c->render_tree != 0 ? 1u : 0u;
+        a.group = group ? 1u : 0u;
         a.totals = count_fetches ? jobs[0].scene->totals.as<unsigned long long>() : nullptr;
         a.spill = w.spill.as<uint32_t>();
         a.spill_stride = (uint32_t)(std::max(ext_grid, graph ? graph_tail_grid : tail_grid) * extend_block());
@@ -750,7 +859,9 @@ Status render_jobs(aurora_ctx* c, std::vector<Job>& jobs, aurora_render_stats* s
                 }
                 break;
             }
-            const int eg = (int)std::min<uint64_t>((uint64_t)ext_grid, blocks);
+            const uint64_t eblocks = group ? std::max<uint64_t>(1, ((uint64_t)ub + kGroupBlockRays - 1) / kGroupBlockRays)
+                                           : blocks;
+            const int eg = (int)std::min<uint64_t>((uint64_t)ext_grid, eblocks);
             const int sg = (int)std::min<uint64_t>((uint64_t)c->shade_grid, blocks);
             ExtendArgs a = extend_args(cur);
             hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -1079,6 +1190,16 @@ int aurora_bvh_download_wide(aurora_scene* s, aurora_bvh4_node* nodes, uint32_t 
     CK(c, hip_status(hipMemcpyAsync(nodes, s->wide.p, (size_t)n * 128, hipMemcpyDeviceToHost, c->stream),
                      "hipMemcpyAsync"));
     CK(c, hip_status(hipStreamSynchronize(c->stream), "hipStreamSynchronize"));
+    // device order (four lower bounds, then four upper ones) to slot order
+    static_assert(sizeof(aurora_bvh4_node) == 128 && sizeof(aurora_bvh4_slot) == 32, "four-wide node layout");
+    for (uint32_t i = 0; i < n; ++i) {
+        float4 dev[8];
+        memcpy(dev, &nodes[i], sizeof dev);
+        for (int k = 0; k < 4; ++k) {
+            memcpy(&nodes[i].slot[k], &dev[k], 16);
+            memcpy(reinterpret_cast<unsigned char*>(&nodes[i].slot[k]) + 16, &dev[4 + k], 16);
+        }
+    }
     return AURORA_OK;
 }
 
@@ -1141,12 +1262,33 @@ int aurora_trace_closest_device_noalloc(aurora_scene* s, const float* o, const f
     SceneRec* rec = reinterpret_cast<SceneRec*>(base + kNaOffRec);
     uint32_t* spill = reinterpret_cast<uint32_t*>(base + kNaOffSpill);
     const uint32_t blocks = (n + 255) / 256;
+    if (!counts) {
+        if (hits_over_rays(o, d, prim, t, n)) {
+            k_copy3<<<blocks, 256, 0, c->stream>>>(o, reinterpret_cast<float*>(ro), n);
+            k_copy3<<<blocks, 256, 0, c->stream>>>(d, reinterpret_cast<float*>(rd), n);
+            o = reinterpret_cast<const float*>(ro);
+            d = reinterpret_cast<const float*>(rd);
+        }
+        QueryArgs q{};
+        q.org = o;
+        q.dir = d;
+        q.n = n;
+        q.sc = group_scene(s->view, tmin);
+        q.tmax = tmax;
+        q.pool = pool;
+        q.prim = prim;
+        q.t = t;
+        q.spill = spill;
+        q.spill_stride = (uint32_t)kNoAllocGrid * kExtendBlock;
+        CK(c, launch_query(q, std::min(grid_for_group(c, n), kNoAllocGrid), c->stream));
+        return AURORA_OK;
+    }
     k_pack3<<<blocks, 256, 0, c->stream>>>(o, ro, n);
     k_pack3<<<blocks, 256, 0, c->stream>>>(d, rd, n);
     SceneRec r{};
     r.sc = s->view;
     r.tmin = tmin;
-    k_noalloc_setup<<<1, kPools * kPoolStride, 0, c->stream>>>(pool, rec, r);
+    k_noalloc_setup<<<1, 64, 0, c->stream>>>(pool, rec, r);
     CK(c, hip_status(hipGetLastError(), "allocation-free query setup"));
     ExtendArgs a{};
     a.ray_o = ro;

@@ -57,6 +57,10 @@ __device__ __forceinline__ v3 refract(v3 uv, v3 n, float eta) {
     return perp + pl * n;
 }
 __device__ __forceinline__ v3 xyz(float4 a) { return v3{a.x, a.y, a.z}; }
+__device__ __forceinline__ v3 load3(const float* p, size_t i) {
+    const float* q = p + 3 * i;
+    return v3{q[0], q[1], q[2]};
+}
 __device__ __forceinline__ v3 clamp01(v3 a) {
     return v3{fminf(fmaxf(a.x, 0.0f), 1.0f), fminf(fmaxf(a.y, 0.0f), 1.0f), fminf(fmaxf(a.z, 0.0f), 1.0f)};
 }

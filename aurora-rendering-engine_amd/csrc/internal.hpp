@@ -11,8 +11,9 @@
 
 namespace aur {
 
-// extend work pools: one counter per XCD, each on its own 128-byte line
-constexpr int kPools = 8;
+// work pools: one counter per range of the items, each on its own 128-byte
+// line (WaveClaims, traverse.hpp)
+constexpr int kPools = 64;
 constexpr uint32_t kPoolStride = 32;
 // render counters: [0], [1] queue counts, pools from kPoolBase
 constexpr uint32_t kPoolBase = 32;
@@ -130,6 +131,7 @@ struct ExtendArgs {
     const struct SceneRec* recs;  // scene table; a ray's scene is the bits of ray_d.w
     uint32_t one_scene;       // nonzero: every ray belongs to recs[0]
     uint32_t wide;            // nonzero: walk the four-wide tree, else the binary one
+    uint32_t group;           // nonzero: four-wide without counters by the group walk, else one lane per ray
     const uint32_t* order;    // optional: claim order of the rays (slot -> ray index)
     uint32_t* counts;         // optional: 3 per ray (nodes, spheres, quads fetched)
     unsigned long long* totals; // optional: [nodes, spheres, quads] summed
@@ -137,12 +139,33 @@ struct ExtendArgs {
     uint32_t spill_stride;    // threads in the persistent grid
 };
 Status launch_extend(const ExtendArgs& a, int grid, hipStream_t stream);
+// The scene of a group walk (traverse.hpp).
+struct GroupScene {
+    const float4 *wide, *spheres, *quads;
+    uint32_t n_wide, n_spheres, n_prims;
+    float tmin;
+};
+constexpr int kGroupBlockRays = 64;  // rays that a block of a group walk holds
+// Closest hits of n rays given as packed floats, into prim and t.
+struct QueryArgs {
+    const float *org, *dir;   // 3 per ray
+    uint32_t n;
+    GroupScene sc;
+    float tmax;
+    const uint32_t* order;    // optional: claim order of the rays (slot -> ray index)
+    uint32_t* pool;           // kPools work counters kPoolStride u32 apart (set to 0 by launch_query when used)
+    int32_t* prim;
+    float* t;
+    uint32_t* spill;          // as in ExtendArgs
+    uint32_t spill_stride;
+};
+Status launch_query(const QueryArgs& a, int grid, hipStream_t stream);
 Status launch_brute(const DevScene& sc, const float4* o, const float4* d, uint32_t n, float tmin, float tmax,
                     float2* hit, hipStream_t stream);
 // Sort keys of n rays for traversal order: 27-bit Morton code of the origin
 // within the box of the scene's root node (origins outside are clamped),
 // then the 3-bit direction octant; values are the ray indices.
-Status launch_ray_keys(const float4* ray_o, const float4* ray_d, uint32_t n, const float4* nodes, uint32_t* keys,
+Status launch_ray_keys(const float* org, const float* dir, uint32_t n, const float4* nodes, uint32_t* keys,
                        uint32_t* vals, hipStream_t stream);
 int extend_block();         // threads per block of the extend kernel
 int extend_spill_levels();  // u32 stack entries per thread in ExtendArgs::spill

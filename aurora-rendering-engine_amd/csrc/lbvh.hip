@@ -622,10 +622,14 @@ __global__ __launch_bounds__(kBlock) void k_wide_reset(uint32_t n, uint32_t* wfl
     if (i == 0) *maxlv = 0u;
 }
 
+// A node on the device holds its four slots' (lo, ref) and then their
+// (hi, 0), 64 bytes each, so that four lanes that read one slot each read
+// consecutive bytes (the group walk); aurora_bvh_download_wide interleaves
+// them into aurora_bvh4_node.
 __device__ __forceinline__ void wide_slot(float4* w, int k, const float4* nodes, uint32_t pos, uint32_t ref) {
     const float4 lo = nodes[2 * (size_t)pos], hi = nodes[2 * (size_t)pos + 1];
-    w[2 * k] = make_float4(lo.x, lo.y, lo.z, __uint_as_float(ref));
-    w[2 * k + 1] = make_float4(hi.x, hi.y, hi.z, 0.0f);
+    w[k] = make_float4(lo.x, lo.y, lo.z, __uint_as_float(ref));
+    w[4 + k] = make_float4(hi.x, hi.y, hi.z, 0.0f);
 }
 
 // one wide node per flagged internal node i, at widx[i] (the exclusive scan
@@ -642,8 +646,8 @@ __global__ __launch_bounds__(kBlock) void k_wide_fill(uint32_t ni, const uint32_
     for (int q = 0; q < m; ++q)
         wide_slot(w, q, nodes, r[q].pos, r[q].leaf ? __float_as_uint(nodes[2 * (size_t)r[q].pos].w) : widx[r[q].j]);
     for (int q = m; q < 4; ++q) {
-        w[2 * q] = make_float4(0.0f, 0.0f, 0.0f, __uint_as_float(AURORA_BVH4_EMPTY));
-        w[2 * q + 1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        w[q] = make_float4(0.0f, 0.0f, 0.0f, __uint_as_float(AURORA_BVH4_EMPTY));
+        w[4 + q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
 }
 
@@ -654,8 +658,8 @@ __global__ void k_wide_single(const float4* nodes, float4* wide) {
     if (k == 0) {
         wide_slot(wide, 0, nodes, 0, __float_as_uint(nodes[0].w));
     } else {
-        wide[2 * k] = make_float4(0.0f, 0.0f, 0.0f, __uint_as_float(AURORA_BVH4_EMPTY));
-        wide[2 * k + 1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        wide[k] = make_float4(0.0f, 0.0f, 0.0f, __uint_as_float(AURORA_BVH4_EMPTY));
+        wide[4 + k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
 }
 

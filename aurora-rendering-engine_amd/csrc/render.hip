@@ -26,12 +26,6 @@ namespace {
 
 constexpr int kBlock = 256;
 
-// The number of lanes below this one whose bit is set in mask (v_mbcnt:
-// a ballot rank without a per-lane mask register).
-__device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-}
-
 // The scene record of a path.  A single-scene launch reads recs[0] through
 // the constant address space: nothing writes the table while a render
 // kernel runs, so its fields arrive by scalar loads and the scene's pointers
@@ -190,10 +184,6 @@ __device__ __forceinline__ void store3(float* p, uint32_t path, v3 v) {
     q[0] = v.x;
     q[1] = v.y;
     q[2] = v.z;
-}
-__device__ __forceinline__ v3 load3(const float* p, size_t i) {
-    const float* q = p + 3 * i;
-    return V(q[0], q[1], q[2]);
 }
 
 struct ShadeBufs {
@@ -408,10 +398,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(TREE == 
     const uint32_t n = b.counters[b.cur];
     uint32_t* my_spill = spill + (size_t)blockIdx.x * kBlock + threadIdx.x;
     const int lane = threadIdx.x & 63;
-    // the queue is split into one contiguous range per XCD; a wave whose
+    // the queue is split into one contiguous range per XCD, with a counter
+    // each (WaveClaims' 64 counters cost this kernel's register budget more
+    // than its claims of 64-128 paths wait: Cornell 7.37 -> 7.54 ms); a wave whose
     // range is spent moves on to the next ones, so uneven ranges (a batch's
     // scenes differ in cost per path) still finish together
-    const uint32_t parts = min((uint32_t)kPools, gridDim.x);
+    const uint32_t parts = min(8u, gridDim.x);
     uint32_t part = blockIdx.x % parts, spent = 0;
     uint32_t r_lo = (uint32_t)(((uint64_t)n * part) / parts);
     uint32_t r_n = (uint32_t)(((uint64_t)n * (part + 1)) / parts) - r_lo;

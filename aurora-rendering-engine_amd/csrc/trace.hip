@@ -1,16 +1,30 @@
 // trace.hip — closest-hit traversal of the LBVH on gfx950 (the extend phase
 // of the wavefront path tracer and the parity entry aurora_trace_closest).
 //
-// k_extend is persistent: a grid sized to the resident capacity of the chip
-// pulls rays from a global pool.  Each lane owns one ray; when enough lanes
-// of a wave64 have finished, the wave claims that many new rays with one
-// atomic and hands them out by ballot prefix (refilling idle lanes).  The
-// rays walk the four-wide tree collapsed from the LBVH: one step fetches a
-// 128-byte node (one cache line, four child boxes), tests the four slabs,
-// intersects leaf primitives at once and descends to the nearest hit child,
-// pushing the others farthest first.  The stack lives in LDS (kLds entries
-// per lane, laid out [level][thread] so a wave's pushes hit 64 consecutive
-// banks) and spills deeper levels to a per-thread global array.
+// Two persistent kernels, both over grids sized to the resident capacity of
+// the chip, whose waves claim rays from WaveClaims' counters:
+//   k_query / k_extend_group  the group walk (traverse.hpp): four lanes per ray
+//     on the four-wide tree.  Every uncounted ray query, and the bounces of
+//     renders of larger scenes.
+//   k_extend  one lane per ray: the binary tree (render bounces), the four-wide
+//     tree for small scenes' bounces, and every run that counts fetches (their
+//     counts are those of this visit order).  When enough lanes of a wave64
+//     have finished, the wave hands out new rays by ballot rank.  A four-wide
+//     step fetches a 128-byte node (one cache line, four child boxes), tests
+//     the four slabs, intersects leaf primitives at once and descends to the
+//     nearest hit child, pushing the others farthest first.  The stack lives in
+//     LDS (kLds entries per lane, laid out [level][thread] so a wave's pushes
+//     hit 64 consecutive banks) and spills deeper levels to a per-thread global
+//     array.
+//
+// What the group walk gave (queries, one lane per ray before -> after): 2^20
+// sorted rays on 1.2 M overlapping primitives 11.9 -> 6.2 ms; 10^6 rays on 190 k
+// primitives 0.70 -> 0.51 ms, on 488 spheres 0.24 -> 0.15; 10^5 rays on 50 k
+// primitives 210 -> 115 us; 1000 rays 57 -> 13 us (of which the packing kernels
+// and the upload of a scene record, with its synchronisation, were 40).  It is
+// bound by VALU issue (one wave instruction per SIMD and 4 cycles: 4.26e9 in
+// 6.6 ms, with 52 of 64 lanes active; 27 of 64 before, when the L1 address path
+// was busy 75% of the time).
 //
 // Reference counterpart: the per-ray linear scan over all triangles,
 // experiments/rt.cpp:209-218, with are::Triangle::intersect_ray
@@ -26,7 +40,6 @@ constexpr int kBlock = 256;
 constexpr int kLds = 16;
 constexpr int kMaxStack = 96;  // three pushes per level of a tree of depth <= 64
 constexpr int kRefill = 8;
-constexpr int kParts = 8;
 constexpr uint32_t kNone = 0xffffffffu;
 constexpr uint32_t kNoPrim = 0x7fffffffu;
 
@@ -43,7 +56,6 @@ __global__ __launch_bounds__(kBlock) void k_extend(ExtendArgs a) {
     if (a.zero_after && blockIdx.x == 0 && threadIdx.x == 0) *a.zero_after = 0u;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     uint32_t* spill = a.spill + (size_t)blockIdx.x * kBlock + tid;
     const size_t sstride = a.spill_stride;
     const float tmax = a.tmax;
@@ -111,57 +123,21 @@ __global__ __launch_bounds__(kBlock) void k_extend(ExtendArgs a) {
         ri = kNone;
     };
 
-    // Work distribution: the rays are split into up to kParts contiguous
-    // ranges, one per XCD (blocks are dealt to the 8 XCDs round-robin), each
-    // with its own pool counter on its own 128-byte line.  A wave claims a
-    // batch of its range with one atomic and deals it out to idle lanes by
-    // ballot rank; a plain load skips the atomic once the range is spent.
-    // A wave whose range is spent moves on to the next ones, so uneven
-    // ranges still finish together.
-    const uint32_t parts = min((uint32_t)kParts, gridDim.x);
-    uint32_t part = blockIdx.x % parts, spent = 0;
-    uint32_t r_lo = (uint32_t)(((uint64_t)n * part) / parts);
-    uint32_t r_n = (uint32_t)(((uint64_t)n * (part + 1)) / parts) - r_lo;
-    uint32_t* pool = a.pool + kPoolStride * part;
-    const uint32_t waves = ((gridDim.x - part + parts - 1) / parts) * (kBlock / 64);
-    // about an eighth of a wave's share of its range per claim: half a share
-    // left the last claims unbalanced (2^22 sorted stress queries: 146 ms
-    // against 126 ms with eighths; 32nds measured the same as eighths)
-    const uint32_t batch = min(4096u, max(64u, r_n / (waves * 8u) + 1u));
-    uint32_t b_next = 0, b_end = 0;  // wave-uniform, offsets within the range
+    WaveClaims claims;
+    claims.init(a.pool, n, 64u, 0u);
     for (;;) {
         const bool idle = (ri == kNone) && !done;
         const uint64_t im = __ballot(idle);
         const uint64_t am = __ballot(ri != kNone);
         if (im != 0 && (am == 0 || __popcll(im) >= kRefill)) {
-            // at most `parts` ranges are tried, each once after it is spent
-            while (b_next >= b_end && spent < parts) {
-                uint32_t base = r_n;
-                if (lane == 0) {
-                    if (__hip_atomic_load(pool, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < r_n)
-                        base = atomicAdd(pool, batch);
-                }
-                // every lane of the wave is active here (no lane leaves the
-                // loop before the whole wave does), so lane 0 is the first
-                // active lane; a scalar copy keeps the range state in SGPRs
-                base = __builtin_amdgcn_readfirstlane(base);
-                if (base < r_n) {
-                    b_next = base;
-                    b_end = min(r_n, base + batch);
-                } else if (++spent < parts) {
-                    part = part + 1 == parts ? 0u : part + 1;
-                    r_lo = (uint32_t)(((uint64_t)n * part) / parts);
-                    r_n = (uint32_t)(((uint64_t)n * (part + 1)) / parts) - r_lo;
-                    pool = a.pool + kPoolStride * part;
-                }
-            }
-            const uint32_t avail = b_next < b_end ? b_end - b_next : 0u;
-            const uint32_t rank = (uint32_t)__popcll(im & lt);
+            claims.refill();
+            const uint32_t avail = claims.next < claims.end ? claims.end - claims.next : 0u;
+            const uint32_t rank = lanes_below(im);
             if (idle) {
                 if (avail == 0) {
                     done = true;
                 } else if (rank < avail) {
-                    ri = r_lo + b_next + rank;
+                    ri = claims.next + rank;
                     if (a.order) ri = a.order[ri];
                     const float4 ro = a.ray_o[ri], rd = a.ray_d[ri];
                     o = xyz(ro);
@@ -201,7 +177,7 @@ __global__ __launch_bounds__(kBlock) void k_extend(ExtendArgs a) {
                     }
                 }
             }
-            b_next += min(avail, (uint32_t)__popcll(im));
+            claims.next += min(avail, (uint32_t)__popcll(im));
         }
         if (__ballot((ri != kNone) || !done) == 0) break;
         if (ri == kNone) continue;
@@ -293,6 +269,144 @@ __global__ __launch_bounds__(kBlock) void k_extend(ExtendArgs a) {
     }
 }
 
+constexpr int kGroupFlush = 48;   // lanes with a leaf before leaves are tested (32: 6848, 40: 6761, 48: 6754 us)
+
+
+// Closest hits over the four-wide tree by the group walk.  IO names the rays,
+// their scenes and where the hits go.  A wave fetches kGroupBatch rays at a
+// time, one per lane and one batch ahead, and keeps them in shared memory for
+// its groups: fetched by the group that takes it, each ray stopped all 16
+// walks for a memory latency (short walks then ran at a quarter of the speed).
+constexpr int kGroupBatch = 16;   // 32 and 64 leave room for fewer waves (sorted queries 6.6, 7.0, 7.8 ms)
+struct QueryShared {
+    GroupShared g;
+    float ray[9][kGroupBatch];
+    uint32_t id[kGroupBatch], scene[kGroupBatch];
+};
+template <class IO>
+__device__ __forceinline__ void group_trace(const IO& io, uint32_t n, uint32_t* pool, float tmax, uint32_t* spill,
+                                            uint32_t spill_stride) {
+    __shared__ QueryShared shared[kBlock / 64];
+    const int lane = threadIdx.x & 63, ray = lane >> 2, slot = lane & 3;
+    QueryShared& sh = shared[threadIdx.x >> 6];
+    const size_t stride = spill_stride / 4;
+    GroupWalk w;
+    group_init(w, sh.g, spill + 2 * (size_t)(blockIdx.x * kGroupBlockRays + (threadIdx.x >> 2)), ray, slot);
+    GroupScene sc = io.scene();
+    WaveClaims claims;
+    claims.init(pool, n, kGroupRays, 0u);
+    uint32_t ri = kNone;
+    uint32_t head = 0, tail = 0;  // the batch's rays not yet taken
+    // the next batch, in registers
+    v3 no = V(0, 0, 0), nd = V(0, 0, 0);
+    uint32_t ni = 0, ns = 0, n_next = 0;
+    auto fetch = [&]() {
+        claims.refill();
+        n_next = claims.next < claims.end ? min(claims.end - claims.next, (uint32_t)kGroupBatch) : 0u;
+        if ((uint32_t)lane < n_next) ni = io.ray(claims.next + lane, no, nd, ns);
+        claims.next += n_next;
+    };
+    fetch();
+    for (;;) {
+        const uint64_t im = __ballot(ri == kNone);
+        if (im != 0) {
+            if (head == tail && n_next != 0) {
+                if ((uint32_t)lane < n_next) {
+                    sh.ray[0][lane] = no.x;
+                    sh.ray[1][lane] = no.y;
+                    sh.ray[2][lane] = no.z;
+                    sh.ray[3][lane] = nd.x;
+                    sh.ray[4][lane] = nd.y;
+                    sh.ray[5][lane] = nd.z;
+                    sh.ray[6][lane] = rcp_rn(nd.x);
+                    sh.ray[7][lane] = rcp_rn(nd.y);
+                    sh.ray[8][lane] = rcp_rn(nd.z);
+                    sh.id[lane] = ni;
+                    if constexpr (!IO::kOneScene) sh.scene[lane] = ns;
+                }
+                head = 0;
+                tail = n_next;
+                group_sync();
+                fetch();
+            }
+            if (head < tail) {
+                const uint32_t at = head + (lanes_below(im) >> 2);
+                if (ri == kNone && at < tail) {
+                    ri = sh.id[at];
+                    if constexpr (!IO::kOneScene) sc = io.scene(sh.scene[at]);
+                    group_begin(w, sh.g, sc, V(sh.ray[0][at], sh.ray[1][at], sh.ray[2][at]),
+                                V(sh.ray[3][at], sh.ray[4][at], sh.ray[5][at]),
+                                V(sh.ray[6][at], sh.ray[7][at], sh.ray[8][at]), tmax, ray, slot);
+                }
+                head = min(tail, head + ((uint32_t)__popcll(im) >> 2));
+            } else if (im == ~0ull) {
+                break;
+            }
+        }
+        group_sync();
+        group_step<IO::kOneScene>(w, sh.g, sc, ray, slot, stride);
+        group_sync();
+        // leaves are tested when enough lanes have one, when a ray has no room
+        // for more, or when no ray can go on without
+        const uint64_t pend = __ballot(group_pending(w, slot));
+        if (pend != 0 && (__popcll(pend) >= kGroupFlush || __ballot(group_full(w)) != 0 ||
+                          __ballot(group_walking(w)) == 0))
+            group_leaves(w, sh.g, sc, tmax, ray, slot);
+        if (w.st == 0u && ri != kNone) {
+            const bool miss = w.best_id == kNoPrim;
+            if (slot == 0) io.hit(ri, miss ? tmax : w.best_t, miss ? AURORA_MISS : (int)w.best_id);
+            ri = kNone;
+        }
+    }
+}
+
+struct QueryIO {
+    static constexpr bool kOneScene = true;
+    const QueryArgs& a;
+    __device__ __forceinline__ GroupScene scene() const { return a.sc; }
+    __device__ __forceinline__ uint32_t ray(uint32_t i, v3& o, v3& d, uint32_t&) const {
+        if (a.order) i = a.order[i];
+        o = load3(a.org, i);
+        d = load3(a.dir, i);
+        return i;
+    }
+    __device__ __forceinline__ void hit(uint32_t i, float t, int prim) const {
+        a.t[i] = t;
+        a.prim[i] = prim;
+    }
+};
+__global__ __launch_bounds__(kBlock) void k_query(QueryArgs a) {
+    group_trace(QueryIO{a}, a.n, a.pool, a.tmax, a.spill, a.spill_stride);
+}
+
+// the live queue of a wavefront bounce
+template <bool ONE>
+struct QueueIO {
+    static constexpr bool kOneScene = ONE;
+    const ExtendArgs& a;
+    __device__ __forceinline__ GroupScene scene() const { return ONE ? group_scene(a.recs[0]) : GroupScene{}; }
+    __device__ __forceinline__ GroupScene scene(uint32_t sid) const { return group_scene(a.recs[sid]); }
+    __device__ __forceinline__ uint32_t ray(uint32_t i, v3& o, v3& d, uint32_t& sid) const {
+        const float4 ro = a.ray_o[i], rd = a.ray_d[i];
+        o = xyz(ro);
+        d = xyz(rd);
+        sid = __float_as_uint(rd.w);
+        return i;
+    }
+    __device__ __forceinline__ void hit(uint32_t i, float t, int prim) const {
+        a.hit[i] = make_float2(t, __int_as_float(prim));
+    }
+};
+template <bool ONE>
+__global__ __launch_bounds__(kBlock) void k_extend_group(ExtendArgs a) {
+    if (a.zero_after && blockIdx.x == 0 && threadIdx.x == 0) *a.zero_after = 0u;
+    group_trace(QueueIO<ONE>{a}, a.count ? *a.count : a.n, a.pool, a.tmax, a.spill, a.spill_stride);
+}
+
+__global__ void k_clear_pool(uint32_t* pool) {
+    if (threadIdx.x < kPools) pool[kPoolStride * threadIdx.x] = 0u;
+}
+
 __global__ __launch_bounds__(kBlock) void k_brute(DevScene sc, const float4* ro, const float4* rd, uint32_t n,
                                                   float tmin, float tmax, float2* hit) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
@@ -344,12 +458,12 @@ __device__ __forceinline__ uint32_t cell9(float x, float lo, float hi) {
     return (uint32_t)fminf(fmaxf(u * 512.0f, 0.0f), 511.0f);
 }
 
-__global__ __launch_bounds__(kBlock) void k_ray_keys(const float4* ro, const float4* rd, uint32_t n,
+__global__ __launch_bounds__(kBlock) void k_ray_keys(const float* ro, const float* rd, uint32_t n,
                                                      const float4* nodes, uint32_t* keys, uint32_t* vals) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
     const float4 lo = nodes[0], hi = nodes[1];
-    const float4 o = ro[i], d = rd[i];
+    const v3 o = load3(ro, i), d = load3(rd, i);
     const uint32_t m = (spread9(cell9(o.x, lo.x, hi.x)) << 2) | (spread9(cell9(o.y, lo.y, hi.y)) << 1) |
                        spread9(cell9(o.z, lo.z, hi.z));
     const uint32_t oct = (d.x < 0.0f ? 4u : 0u) | (d.y < 0.0f ? 2u : 0u) | (d.z < 0.0f ? 1u : 0u);
@@ -359,7 +473,7 @@ __global__ __launch_bounds__(kBlock) void k_ray_keys(const float4* ro, const flo
 
 }  // namespace
 
-Status launch_ray_keys(const float4* ro, const float4* rd, uint32_t n, const float4* nodes, uint32_t* keys,
+Status launch_ray_keys(const float* ro, const float* rd, uint32_t n, const float4* nodes, uint32_t* keys,
                        uint32_t* vals, hipStream_t s) {
     if (n == 0) return Status::ok();
     k_ray_keys<<<(n + kBlock - 1) / kBlock, kBlock, 0, s>>>(ro, rd, n, nodes, keys, vals);
@@ -367,9 +481,9 @@ Status launch_ray_keys(const float4* ro, const float4* rd, uint32_t n, const flo
     return Status::ok();
 }
 
-static_assert(kExtendBlock == kBlock && kExtendSpillLevels == kMaxStack - kLds, "extend shape constants");
+static_assert(kExtendBlock == kBlock && kExtendSpillLevels >= kMaxStack - kLds, "extend shape constants");
 int extend_block() { return kBlock; }
-int extend_spill_levels() { return kMaxStack - kLds; }
+int extend_spill_levels() { return kExtendSpillLevels; }
 
 Status launch_extend(const ExtendArgs& a, int grid, hipStream_t s) {
     if ((size_t)grid * kBlock > a.spill_stride) return Status{AURORA_ERR_RUNTIME, "extend grid exceeds spill stride"};
@@ -379,7 +493,25 @@ Status launch_extend(const ExtendArgs& a, int grid, hipStream_t s) {
                                        k_extend<false, true, false>,  k_extend<false, true, true>,
                                        k_extend<true, false, false>,  k_extend<true, false, true>,
                                        k_extend<true, true, false>,   k_extend<true, true, true>};
-    ks[v]<<<grid, kBlock, 0, s>>>(a);
+    if (a.group && a.wide && !count) {
+        auto k = a.one_scene ? k_extend_group<true> : k_extend_group<false>;
+        k<<<grid, kBlock, 0, s>>>(a);
+    } else {
+        ks[v]<<<grid, kBlock, 0, s>>>(a);
+    }
+    AUR_HIP(hipGetLastError());
+    return Status::ok();
+}
+
+Status launch_query(const QueryArgs& args, int grid, hipStream_t s) {
+    QueryArgs a = args;
+    if ((size_t)grid * kBlock > a.spill_stride) return Status{AURORA_ERR_RUNTIME, "query grid exceeds spill stride"};
+    if ((uint64_t)grid * kGroupBlockRays >= a.n) {
+        a.pool = nullptr;  // one ray per place: nothing to claim
+    } else {
+        k_clear_pool<<<1, 64, 0, s>>>(a.pool);
+    }
+    k_query<<<grid, kBlock, 0, s>>>(a);
     AUR_HIP(hipGetLastError());
     return Status::ok();
 }
