@@ -81,8 +81,7 @@ int aurora_denoise(aurora_denoiser* d, const float* rgb, const float* alb, const
     if (!rgb || !alb || !nrm || !out || spp == 0)
         return ctx_fail(d->ctx, AURORA_ERR_INVALID, "NULL buffer or spp == 0");
     DCK(d, set_device(d));
-    DCK(d, d->net->forward(rgb, alb, nrm, 1.0f / (float)spp, 1, (int)height, (int)width));
-    DCK(d, d->net->write_output(out));
+    DCK(d, d->net->forward(rgb, alb, nrm, 1.0f / (float)spp, 1, (int)height, (int)width, out));
     return AURORA_OK;
 }
 
@@ -101,7 +100,7 @@ int aurora_denoiser_loss_grad(aurora_denoiser* d, const float* rgb, const float*
     if (!rgb || !alb || !nrm || !target || spp == 0 || batch == 0)
         return ctx_fail(d->ctx, AURORA_ERR_INVALID, "NULL buffer, spp == 0 or batch == 0");
     DCK(d, set_device(d));
-    DCK(d, d->net->forward(rgb, alb, nrm, 1.0f / (float)spp, (int)batch, (int)height, (int)width));
+    DCK(d, d->net->forward(rgb, alb, nrm, 1.0f / (float)spp, (int)batch, (int)height, (int)width, nullptr));
     DCK(d, d->net->backward(target, loss));
     if (host_grads) DCK(d, d->net->grads_to_host(host_grads));
     return AURORA_OK;

@@ -107,7 +107,7 @@ Status Unet::alloc(int N, int H, int W) {
     if (N == N_ && H == H_ && W == W_) return Status::ok();
     for (int s = 0; s < kSlots; ++s) {
         const size_t cnt = (size_t)N * (H >> slot_lv_[s]) * (W >> slot_lv_[s]) * slot_c_[s];
-        AUR_TRY(act_[s].alloc(cnt * (s == kOut ? 4 : 2)));
+        AUR_TRY(act_[s].alloc(s == kOut ? (size_t)N * H * W * 3 * 4 : cnt * 2));
     }
     AUR_TRY(noisy_log_.alloc((size_t)N * H * W * 3 * 4));
     AUR_TRY(loss_part_.alloc(((size_t)N * H * W + 255) / 256 * 4 + 16));
@@ -117,76 +117,97 @@ Status Unet::alloc(int N, int H, int W) {
     return Status::ok();
 }
 
-Status Unet::forward(const float* rgb, const float* alb, const float* nrm, float inv_spp, int N, int H, int W) {
+Status Unet::forward(const float* rgb, const float* alb, const float* nrm, float inv_spp, int N, int H, int W,
+                     float* img) {
     if (N < 1 || H < 8 || W < 8 || (H % 8) || (W % 8))
         return Status{AURORA_ERR_INVALID, "denoiser: image height and width must be positive multiples of 8"};
     AUR_TRY(alloc(N, H, W));
     const size_t npix = (size_t)N * H * W;
     AUR_TRY(prep_input(rgb, alb, nrm, npix, inv_spp, act_[0].as<uint16_t>(), noisy_log_.as<float>(), s_));
-    for (size_t li = 0; li < layers_.size(); ++li) {
-        const Layer& L = layers_[li];
-        // pooled inputs are produced just before the first layer that reads them
+    bool pooled[kSlots] = {};
+    for (const Layer& L : layers_) {
+        const int h = H >> L.level, w = W >> L.level;
+        // a pooled input that the layer before did not write
         for (const auto& pl : kPoolSlots)
-            if (pl[1] == L.a)
-                AUR_TRY(avgpool2(act_[pl[0]].as<uint16_t>(), N, H >> slot_lv_[pl[0]], W >> slot_lv_[pl[0]],
-                                 slot_c_[pl[0]], act_[pl[1]].as<uint16_t>(), s_));
+            if (pl[1] == L.a && !pooled[L.a])
+                AUR_TRY(avgpool2(act_[pl[0]].as<uint16_t>(), N, 2 * h, 2 * w, slot_c_[pl[0]],
+                                 act_[pl[1]].as<uint16_t>(), s_));
         ConvIn in{act_[L.a].as<uint16_t>(), L.b >= 0 ? act_[L.b].as<uint16_t>() : nullptr, L.ca, L.cb};
-        const bool f32 = L.out == kOut;
-        AUR_TRY(conv3x3_forward(in, L.wk.as<uint16_t>(), L.kpad, params_.as<float>() + L.b_off, act_[L.out].p, f32,
-                                false, L.relu, N, H >> L.level, W >> L.level, L.cout, s_));
+        const float* bias = params_.as<float>() + L.b_off;
+        if (L.out == kOut) {
+            AUR_TRY(conv_residual(in, L.wk.as<uint16_t>(), bias, img ? noisy_log_.as<float>() : nullptr,
+                                  img ? img : act_[kOut].as<float>(), N, h, w, s_));
+            continue;
+        }
+        uint16_t* pool = nullptr;
+        for (const auto& pl : kPoolSlots)
+            if (pl[0] == L.out && conv_pools(N, h, w)) {
+                pool = act_[pl[1]].as<uint16_t>();
+                pooled[pl[1]] = true;
+            }
+        AUR_TRY(conv_relu(in, L.wk.as<uint16_t>(), bias, act_[L.out].as<uint16_t>(), pool, N, h, w, L.cout, s_));
     }
     return Status::ok();
 }
 
-Status Unet::write_output(float* img) {
-    return output_image(act_[kOut].as<float>(), noisy_log_.as<float>(), (size_t)N_ * H_ * W_, img, s_);
-}
-
+// From the output layer back.  A layer's output gradient is ready in BF16,
+// masked by its ReLU, when the layer is reached: its data-gradient convolution
+// writes its input's directly, except where two gradients are summed first (a
+// skip connection with a pooled copy) or a 2x2 block is (an upsampled input).
+// The weight gradients need only activations and these gradients, and are
+// taken together at the end.
 Status Unet::backward(const float* target, float* loss) {
     const int N = N_, H = H_, W = W_;
     const size_t npix = (size_t)N * H * W;
-    size_t max_cat = 0, max_act = 0;
-    for (int s = 0; s < kSlots; ++s) {
-        const size_t cnt = (size_t)N * (H >> slot_lv_[s]) * (W >> slot_lv_[s]) * slot_c_[s];
-        AUR_TRY(grad_[s].alloc(cnt * 4));
-        AUR_HIP(hipMemsetAsync(grad_[s].p, 0, cnt * 4, s_));
-        max_act = std::max(max_act, cnt);
-    }
+    auto count = [&](int s) { return (size_t)N * (H >> slot_lv_[s]) * (W >> slot_lv_[s]) * slot_c_[s]; };
+    for (const Layer& L : layers_) AUR_TRY(grad_[L.out].alloc(count(L.out) * 2));
+    size_t max_up = 0;
     for (const Layer& L : layers_)
-        if (L.b >= 0) max_cat = std::max(max_cat, (size_t)N * (H >> L.level) * (W >> L.level) * (L.ca + L.cb));
-    AUR_TRY(gbf_.alloc(max_act * 2));
-    AUR_TRY(dcat_.alloc(max_cat * 4));
+        if (L.b >= 0) {
+            AUR_TRY(fgrad_[L.a].alloc(count(L.a) * 4));
+            max_up = std::max(max_up, (size_t)N * (H >> L.level) * (W >> L.level) * L.cb);
+        }
+    AUR_TRY(dup_.alloc(max_up * 4));
+    for (const auto& pl : kPoolSlots) AUR_TRY(fgrad_[pl[1]].alloc(count(pl[1]) * 4));
     AUR_TRY(grads_.alloc(n_params_ * 4));
     const unsigned nb = (unsigned)((npix + 255) / 256);
     AUR_TRY(loss_grad(act_[kOut].as<float>(), noisy_log_.as<float>(), target, npix, loss_kind_,
-                      grad_[kOut].as<float>(), loss_part_.as<float>(), s_));
+                      grad_[kOut].as<uint16_t>(), loss_part_.as<float>(), s_));
+    std::vector<DwPart> parts;
     for (int li = (int)layers_.size() - 1; li >= 0; --li) {
         const Layer& L = layers_[li];
-        const int h = H >> L.level, w = W >> L.level;
-        const size_t cnt = (size_t)N * h * w * L.cout;
-        AUR_TRY(mask_to_bf16(grad_[L.out].as<float>(), L.relu ? act_[L.out].as<uint16_t>() : nullptr, cnt,
-                             gbf_.as<uint16_t>(), s_));
-        ConvIn in{act_[L.a].as<uint16_t>(), L.b >= 0 ? act_[L.b].as<uint16_t>() : nullptr, L.ca, L.cb};
-        AUR_TRY(conv3x3_weight_grad(in, gbf_.as<uint16_t>(), L.cout, N, h, w, grads_.as<float>() + L.w_off,
-                                    grads_.as<float>() + L.b_off, scratch_, s_));
+        const int h = H >> L.level, w = W >> L.level, cin = L.ca + L.cb;
+        const uint16_t* g = grad_[L.out].as<uint16_t>();
+        float* dw = grads_.as<float>() + L.w_off;
+        parts.push_back(DwPart{act_[L.a].as<uint16_t>(), g, L.ca, L.cout, cin, 0, false, N, h, w, dw,
+                               grads_.as<float>() + L.b_off});
+        if (L.b >= 0)
+            parts.push_back(
+                DwPart{act_[L.b].as<uint16_t>(), g, L.cb, L.cout, cin, L.ca, true, N, h, w, dw, nullptr});
         if (li == 0) break;  // no gradient for the network input
-        ConvIn gin{gbf_.as<uint16_t>(), nullptr, L.cout, 0};
-        const int cin = L.ca + L.cb;
-        if (L.b < 0) {
-            AUR_TRY(conv3x3_forward(gin, L.wt.as<uint16_t>(), L.kpad_t, nullptr, grad_[L.a].p, true, true, false, N, h,
-                                    w, cin, s_));
-        } else {
-            AUR_TRY(conv3x3_forward(gin, L.wt.as<uint16_t>(), L.kpad_t, nullptr, dcat_.p, true, false, false, N, h, w,
-                                    cin, s_));
-            AUR_TRY(split_concat_grad(dcat_.as<float>(), N, h, w, L.ca, L.cb, grad_[L.a].as<float>(),
-                                      grad_[L.b].as<float>(), true, s_));
+        const uint16_t* wt = L.wt.as<uint16_t>();
+        if (L.b >= 0) {
+            AUR_TRY(conv_data_grad_f32(g, L.cout, wt, fgrad_[L.a].as<float>(), N, h, w, L.ca, s_));
+            AUR_TRY(conv_data_grad_f32(g, L.cout, wt + (size_t)L.ca * L.kpad_t, dup_.as<float>(), N, h, w, L.cb, s_));
+            AUR_TRY(upsample_grad(dup_.as<float>(), act_[L.b].as<uint16_t>(), N, h, w, L.cb,
+                                  grad_[L.b].as<uint16_t>(), s_));
+            continue;
         }
-        // a pooled slot's gradient is complete once its only reader is done
+        int skip = -1;  // the slot whose pooled copy this layer reads
         for (const auto& pl : kPoolSlots)
-            if (pl[1] == L.a)
-                AUR_TRY(avgpool2_backward(grad_[pl[1]].as<float>(), N, H >> slot_lv_[pl[0]], W >> slot_lv_[pl[0]],
-                                          slot_c_[pl[0]], grad_[pl[0]].as<float>(), s_));
+            if (pl[1] == L.a) skip = pl[0];
+        if (skip < 0) {
+            AUR_TRY(conv_data_grad(g, L.cout, wt, act_[L.a].as<uint16_t>(), grad_[L.a].as<uint16_t>(), N, h, w, cin, s_));
+        } else {
+            AUR_TRY(conv_data_grad_f32(g, L.cout, wt, fgrad_[L.a].as<float>(), N, h, w, cin, s_));
+            AUR_TRY(skip_grad(fgrad_[skip].as<float>(), fgrad_[L.a].as<float>(), act_[skip].as<uint16_t>(), N, 2 * h,
+                              2 * w, slot_c_[skip], grad_[skip].as<uint16_t>(), s_));
+        }
     }
+    size_t floats = 0;
+    for (const DwPart& p : parts) floats += dw_partial_floats(p);
+    AUR_TRY(scratch_.alloc(floats * 4));
+    AUR_TRY(weight_grads(parts.data(), (int)parts.size(), scratch_.as<float>(), s_));
     if (loss) {
         std::vector<float> part(nb);
         AUR_HIP(hipMemcpyAsync(part.data(), loss_part_.p, nb * 4, hipMemcpyDeviceToHost, s_));
@@ -223,10 +244,10 @@ void Unet::release() {
     for (int s = 0; s < kSlots; ++s) {
         act_[s].release();
         grad_[s].release();
+        fgrad_[s].release();
     }
+    dup_.release();
     noisy_log_.release();
-    gbf_.release();
-    dcat_.release();
     scratch_.release();
     loss_part_.release();
 }

@@ -14,25 +14,45 @@ struct ConvIn {
     int ca, cb;
 };
 
-Status conv3x3_forward(const ConvIn& in, const uint16_t* wk, int kpad, const float* bias, void* out, bool out_f32,
-                       bool accum, bool relu, int N, int H, int W, int cout, hipStream_t s);
-Status conv3x3_weight_grad(const ConvIn& in, const uint16_t* g, int cout, int N, int H, int W, float* dw, float* db,
-                           DevBuf& scratch, hipStream_t s);
-Status mask_to_bf16(const float* grad, const uint16_t* act, size_t n, uint16_t* out, hipStream_t s);
+// bias + ReLU; pool: also the 2x2 average of the output (where conv_pools says so)
+Status conv_relu(const ConvIn& in, const uint16_t* w, const float* bias, uint16_t* out, uint16_t* pool, int N, int H,
+                 int W, int cout, hipStream_t s);
+// the size from which conv_relu can pool
+bool conv_pools(int N, int H, int W);
+// the output layer: 3 floats per pixel, the residual, or (noisy given) the image
+// max(expm1(noisy + residual), 0)
+Status conv_residual(const ConvIn& in, const uint16_t* w, const float* bias, const float* noisy, float* out, int N,
+                     int H, int W, hipStream_t s);
+// data gradient of a gradient g of cg channels: BF16 masked by act > 0, or FP32
+Status conv_data_grad(const uint16_t* g, int cg, const uint16_t* w, const uint16_t* act, uint16_t* out, int N, int H,
+                      int W, int cout, hipStream_t s);
+Status conv_data_grad_f32(const uint16_t* g, int cg, const uint16_t* w, float* out, int N, int H, int W, int cout,
+                          hipStream_t s);
+
+// Weight gradient of one layer with respect to one part of its input.
+struct DwPart {
+    const uint16_t *x, *g;  // the part (cx channels; half: at half resolution), the layer's output gradient
+    int cx, cout, cin, ci0; // channels; ci0: the part's first channel in the layer's input of cin
+    bool half;
+    int N, H, W;
+    float *dw, *db;         // [cout][9][cin]; db null: not this part's
+};
+constexpr uint32_t kDwBlocks = 128;  // most blocks, and partial sums, of a part
+size_t dw_partial_floats(const DwPart& p);
+// all parts; scratch holds the sum of their dw_partial_floats
+Status weight_grads(const DwPart* parts, int n, float* scratch, hipStream_t s);
 Status avgpool2(const uint16_t* in, int N, int H, int W, int C, uint16_t* out, hipStream_t s);
-Status avgpool2_backward(const float* gout, int N, int H, int W, int C, float* gin, hipStream_t s);
-Status split_concat_grad(const float* d, int N, int H, int W, int ca, int cb, float* ga, float* gb, bool gb_accum,
-                         hipStream_t s);
+Status upsample_grad(const float* d, const uint16_t* act, int N, int H, int W, int C, uint16_t* g, hipStream_t s);
+Status skip_grad(const float* skip, const float* pool, const uint16_t* act, int N, int H, int W, int C, uint16_t* g,
+                 hipStream_t s);
 Status prep_input(const float* rgb, const float* alb, const float* nrm, size_t npix, float inv_spp, uint16_t* x,
                   float* noisy_log, hipStream_t s);
-Status output_image(const float* out16, const float* noisy_log, size_t npix, float* img, hipStream_t s);
-Status loss_grad(const float* out16, const float* noisy_log, const float* target, size_t npix, int kind,
-                 float* g16f, float* loss_partial, hipStream_t s);
+Status loss_grad(const float* res, const float* noisy_log, const float* target, size_t npix, int kind, uint16_t* g,
+                 float* loss_partial, hipStream_t s);
 Status adam_step(float* w, const float* g, float* m, float* v, size_t n, float lr, float b1, float b2, float eps,
                  int t, hipStream_t s);
 Status pack_weights(const float* w, int cout, int cin, int kpad, int kpad_t, uint16_t* wk, uint16_t* wt,
                     hipStream_t s);
-Status f32_to_bf16(const float* in, size_t n, uint16_t* out, hipStream_t s);
 Status mfma_selftest(const uint16_t* A, const uint16_t* B, float* D, hipStream_t s);
 
 // 4-level U-Net (channels 32/48/64/64), 15 3x3 convolutions.
@@ -53,9 +73,10 @@ class Unet {
     size_t param_count() const { return n_params_; }
     Status get_params(float* host);
     Status set_params(const float* host);
-    // forward on N images of H x W (H, W multiples of 8); out16 kept
-    Status forward(const float* rgb, const float* alb, const float* nrm, float inv_spp, int N, int H, int W);
-    Status write_output(float* img);
+    // forward on N images of H x W (H, W multiples of 8): the denoised image
+    // into img, or (img null) the residual, kept for backward
+    Status forward(const float* rgb, const float* alb, const float* nrm, float inv_spp, int N, int H, int W,
+                   float* img);
     // loss against targets (mean radiance) and gradients into grads_
     Status backward(const float* target, float* loss);
     Status adam(float lr);
@@ -74,9 +95,12 @@ class Unet {
     int t_ = 0;
     int loss_kind_ = 0;
     static constexpr int kSlots = 19;  // x, 14 hidden, 3 pools, out
-    DevBuf act_[kSlots];               // BF16 activations (slot 18: FP32 out16)
-    DevBuf grad_[kSlots];              // FP32 gradients of activations
-    DevBuf noisy_log_, gbf_, dcat_, scratch_, loss_part_;
+    DevBuf act_[kSlots];               // BF16 activations (slot 18: the FP32 residual, 3 per pixel)
+    DevBuf grad_[kSlots];              // BF16 gradients of the layers' outputs, masked by their ReLU
+    // FP32 gradients that are summed with another one: of the skip connections'
+    // and the pooled slots, and of a decoder's upsampled input (full resolution)
+    DevBuf fgrad_[kSlots], dup_;
+    DevBuf noisy_log_, scratch_, loss_part_;
     int slot_c_[kSlots] = {0};
     int slot_lv_[kSlots] = {0};
 };
