@@ -182,7 +182,8 @@ class Context:
 
     def set_render_tree(self, tree=0):
         """Tree the render kernels walk: 0 (or False) the binary LBVH
-        (default), 1 (or True) the four-wide tree, 2 the flat leaf array of a
+        (default; flat for one small scene of large overlapping primitives), 1
+        (or True) the four-wide tree, 2 the flat leaf array of a
         small scene (single-scene renders; four-wide elsewhere).  Speed only;
         the images are the same."""
         self.check(self.lib.aurora_set_render_tree(self.h, int(tree)))

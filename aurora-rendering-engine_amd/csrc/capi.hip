@@ -36,6 +36,7 @@ constexpr uint32_t kSortMinNodes = 1u << 21;
 // 1000 primitives 2.2 -> 2.5, 50 k 7.1 -> 6.4, 190 k 10.4 -> 9.2, 800 k
 // overlapping 10.0 -> 7.4)
 constexpr uint32_t kGroupMinPrims = 16384;
+constexpr uint32_t kFlatDefaultPrims = 64;
 
 struct aurora_ctx {
     int device = 0;
@@ -57,6 +58,7 @@ struct aurora_ctx {
     SceneRec* host_recs[2] = {nullptr, nullptr};
     hipEvent_t recs_ev[2] = {nullptr, nullptr};
     int recs_turn = 0;
+    std::vector<hipEvent_t> cnt_ev;  // wavefront bounces: their live-path counts have arrived
     uint32_t host_recs_cap = 0;
     unsigned char* scratch = nullptr;  // this device's copy of the allocation-free scratch array
     PatchWork patch;                   // patch-projection renderer tables
@@ -70,6 +72,7 @@ struct aurora_scene {
     DevBuf nodes, wide, morton, order, flat;
     BvhScratch scr;
     bool built = false;
+    float flat_overlap = 0.0f;  // flat_build's
     aurora_bvh_stats stats{};
     DevBuf rec1;  // one-entry scene table for ray queries
     DevBuf tr_o, tr_d, tr_hit, tr_spill, tr_pool, totals;
@@ -638,7 +641,16 @@ Status render_jobs(aurora_ctx* c, std::vector<Job>& jobs, aurora_render_stats* s
     // the fused tail is persistent: its grid is the resident capacity
     // the passes walk the flat leaf array under the condition render_jobs
     // sets pa.flat by (one scene, small enough to have the array)
-    const bool flat = c->render_tree == 2 && jobs.size() == 1 && jobs[0].scene->view.n_flat > 0;
+    // (the default tree too where a tree has little to cull: few leaves, whose
+    // boxes a ray enters at least one of on average.  160x120, 1 sample, depth
+    // 8 / 1024x640, 8 samples, depth 50, binary -> flat: the Cornell box, 18
+    // leaves, overlap 2, 215 -> 165 us / 2.41 -> 1.60 ms; scattered scenes of
+    // overlap below 1: 10 leaves 151 -> 143 us / 1.20 -> 1.24 ms, 30 leaves 168 ->
+    // 169 / 1.19 -> 1.25, 120 leaves 202 -> 248 / 1.58 -> 2.07)
+    const bool flat =
+        jobs.size() == 1 && jobs[0].scene->view.n_flat > 0 &&
+        (c->render_tree == 2 || (c->render_tree == 0 && jobs[0].scene->n_prims <= kFlatDefaultPrims &&
+                                 jobs[0].scene->flat_overlap >= 1.0f));
     // four-wide wavefront bounces: the group walk where most paths are in
     // scenes of at least kGroupMinPrims primitives, one lane per ray elsewhere
     uint64_t big = 0, all = 0;
@@ -655,7 +667,10 @@ Status render_jobs(aurora_ctx* c, std::vector<Job>& jobs, aurora_render_stats* s
     AUR_TRY(ensure_workspace(c, (uint32_t)cap, std::max(ext_grid, graph ? graph_tail_grid : tail_grid)));
     Workspace& w = c->ws;
     AUR_TRY(w.recs.alloc(jobs.size() * sizeof(SceneRec)));
-    if (c->host_recs_cap < jobs.size()) {
+    // a single scene's record goes with the raygen launch
+    const bool by_value = jobs.size() == 1 && !graph;
+    SceneRec one_rec{};
+    if (!by_value && c->host_recs_cap < jobs.size()) {
         for (int k = 0; k < 2; ++k) {
             AUR_HIP(hipEventSynchronize(c->recs_ev[k]));  // no copy still reads the old table
             if (c->host_recs[k]) (void)hipHostFree(c->host_recs[k]);
@@ -690,10 +705,8 @@ Status render_jobs(aurora_ctx* c, std::vector<Job>& jobs, aurora_render_stats* s
         AUR_HIP(hipEventRecord(t_begin, c->stream));
     }
     std::vector<hipEvent_t> ext_ev, tail_ev;
-    std::vector<hipEvent_t> cnt_ev(max_depth);
     // counting runs trace every segment in k_extend, whose counters they read
     const uint32_t tail_paths = count_fetches ? 0u : c->tail_paths;
-    for (auto& e2 : cnt_ev) AUR_TRY(ev(e2));
     uint64_t total_segments = 0;
 
     // build the scene table of the next pass; returns its shape
@@ -708,8 +721,12 @@ Status render_jobs(aurora_ctx* c, std::vector<Job>& jobs, aurora_render_stats* s
     auto make_pass = [&](Pass& pa, bool& same_shape, uint32_t& prev_sig, bool& any) -> Status {
         uint32_t path_off = 0, pix_off = 0, sig = 0;
         any = false;
-        AUR_HIP(hipEventSynchronize(c->recs_ev[c->recs_turn]));
-        hrecs = c->host_recs[c->recs_turn];
+        if (by_value) {
+            hrecs = &one_rec;
+        } else {
+            AUR_HIP(hipEventSynchronize(c->recs_ev[c->recs_turn]));
+            hrecs = c->host_recs[c->recs_turn];
+        }
         for (size_t k = 0; k < jobs.size(); ++k) {
             Job& j = jobs[k];
             const uint32_t sp = j.done < j.rd.spp ? std::min(j.S, j.rd.spp - j.done) : 0u;
@@ -759,7 +776,9 @@ Status render_jobs(aurora_ctx* c, std::vector<Job>& jobs, aurora_render_stats* s
     };
     // the kernels add the segments they trace to one device counter over
     // the whole call; it is read once, at the end, and only for statistics
-    AUR_HIP(hipMemsetAsync(w.counters.as<uint32_t>() + kTailSegs, 0, 8, c->stream));
+    // (the first pass's raygen clears it, except in a captured pass, which is replayed)
+    if (graph) AUR_HIP(hipMemsetAsync(w.counters.as<uint32_t>() + kTailSegs, 0, 8, c->stream));
+    bool first_pass = true;
     auto extend_args = [&](int cur) {
         ExtendArgs a{};
         a.ray_o = w.q_o[cur].as<float4>();
@@ -796,7 +815,9 @@ Status render_jobs(aurora_ctx* c, std::vector<Job>& jobs, aurora_render_stats* s
             finish_pass(pa);
             continue;
         }
-        AUR_TRY(stage_recs());
+        if (!by_value) AUR_TRY(stage_recs());
+        pa.first = first_pass && !graph ? 1u : 0u;
+        first_pass = false;
         if (graph) {
             // capture: fixed launch shapes, no host round trips inside
             if (gexec) {
@@ -808,7 +829,7 @@ Status render_jobs(aurora_ctx* c, std::vector<Job>& jobs, aurora_render_stats* s
                 g = nullptr;
             }
             AUR_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-            Status cs = launch_raygen(pa, w, c->stream);
+            Status cs = launch_raygen(pa, nullptr, w, c->stream);
             // captured passes run a fixed number of wavefront bounces, then
             // the fused tail; none when the whole pass fits the tail switch
             const uint32_t dt = pa.n_paths <= tail_paths ? 0u : std::min(max_depth, c->graph_tail_depth);
@@ -830,14 +851,14 @@ Status render_jobs(aurora_ctx* c, std::vector<Job>& jobs, aurora_render_stats* s
             finish_pass(pa);
             continue;
         }
-        AUR_TRY(launch_raygen(pa, w, c->stream));
+        AUR_TRY(launch_raygen(pa, by_value ? &one_rec : nullptr, w, c->stream));
         for (uint32_t depth = 0; depth < max_depth; ++depth) {
             const int cur = depth & 1;
             // queues only shrink, so the count two bounces back bounds this
             // bounce's queue: size both launches from it
             uint32_t ub = pa.n_paths;
             if (depth >= 2) {
-                AUR_HIP(hipEventSynchronize(cnt_ev[depth - 2]));
+                AUR_HIP(hipEventSynchronize(c->cnt_ev[depth - 2]));
                 ub = w.host_counts[depth - 2];
                 if (ub == 0) break;
             }
@@ -879,7 +900,12 @@ Status render_jobs(aurora_ctx* c, std::vector<Job>& jobs, aurora_render_stats* s
             AUR_TRY(launch_shade(pa, w, cur, depth, sg, c->stream));
             AUR_HIP(hipMemcpyAsync(w.host_counts + depth, w.counters.as<uint32_t>() + (cur ^ 1), 4,
                                    hipMemcpyDeviceToHost, c->stream));
-            AUR_HIP(hipEventRecord(cnt_ev[depth], c->stream));
+            while (c->cnt_ev.size() <= depth) {
+                hipEvent_t e = nullptr;
+                AUR_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+                c->cnt_ev.push_back(e);
+            }
+            AUR_HIP(hipEventRecord(c->cnt_ev[depth], c->stream));
         }
         AUR_TRY(launch_accumulate(pa, w, c->stream));
         finish_pass(pa);
@@ -1007,6 +1033,7 @@ void aurora_destroy(aurora_ctx* c) {
     for (DevBuf* b : bufs) b->release();
     c->patch.release();
     if (w.host_counts) (void)hipHostFree(w.host_counts);
+    for (hipEvent_t e : c->cnt_ev) (void)hipEventDestroy(e);
     for (int k = 0; k < 2; ++k) {
         if (c->host_recs[k]) (void)hipHostFree(c->host_recs[k]);
         if (c->recs_ev[k]) (void)hipEventDestroy(c->recs_ev[k]);
@@ -1156,7 +1183,7 @@ int aurora_bvh_build(aurora_scene* s, aurora_bvh_stats* stats) {
     s->view.n_nodes = st.n_nodes;
     s->view.wide = s->wide.as<float4>();
     s->view.n_wide = st.n_nodes ? st.n_wide : 0u;
-    CK(c, flat_build(s->n_prims, s->nodes, s->scr, s->flat, c->stream));
+    CK(c, flat_build(s->n_prims, s->nodes, s->scr, s->flat, c->stream, s->flat_overlap));
     s->view.flat = s->flat.as<float4>();
     s->view.n_flat = s->n_prims <= kFlatMaxPrims ? s->n_prims : 0u;
     s->stats = st;

@@ -105,7 +105,10 @@ Status lbvh_build(const DevScene& sc, uint32_t n_prims, DevBuf& nodes, DevBuf& w
 // Morton order (32 bytes each) for the flat traversal; flat_build fills them
 // from the LBVH that lbvh_build left in `nodes` and `scr`.
 constexpr uint32_t kFlatMaxPrims = 256;
-Status flat_build(uint32_t n_prims, const DevBuf& nodes, const BvhScratch& scr, DevBuf& flat, hipStream_t stream);
+// overlap: the sum of the leaf boxes' areas over the scene box's, about the leaf
+// boxes that a ray through the scene enters.
+Status flat_build(uint32_t n_prims, const DevBuf& nodes, const BvhScratch& scr, DevBuf& flat, hipStream_t stream,
+                  float& overlap);
 
 // Stable LSD radix sort of (key, value) pairs, 8 bits per pass from bit 0.
 // Sorted pairs end in (k0, v0) for an even number of passes, else in
@@ -200,6 +203,7 @@ struct Pass {
     uint32_t wide;         // render traversal over the four-wide tree (else the binary one)
     uint32_t flat;         // the fused tail walks the scene's flat leaf array (one scene with one)
     uint32_t claim;        // paths per work-pool claim in the fused tail (0: by pass size)
+    uint32_t first;        // the call's first pass: raygen clears the segment counter
     uint32_t lean_queue;   // the fused tail carries the pass from the first bounce: raygen writes
                            // directions, and origins for a thin lens only (throughput 1, radiance
                            // set by the tail; a queue position is its path)
@@ -215,7 +219,9 @@ struct Workspace {
     uint32_t capacity = 0;
     uint32_t* host_counts = nullptr;  // pinned, 256 slots
 };
-Status launch_raygen(const Pass& p, Workspace& ws, hipStream_t s);
+// rec: the record of a single-scene pass, which the kernel writes to the table;
+// null: the table is on the device
+Status launch_raygen(const Pass& p, const SceneRec* rec, Workspace& ws, hipStream_t s);
 // camera rays of n (pixel, sample) pairs into 3*n float origins/directions
 // (pixel = j*W + i < W*H, checked by the caller)
 Status launch_camera_rays(const CamF& cam, uint32_t seed, const uint32_t* pixels, const uint32_t* samples,

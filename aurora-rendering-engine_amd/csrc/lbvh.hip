@@ -703,7 +703,9 @@ Status radix_sort_pairs(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, 
 // first (stable: Morton order among equal areas): a flat walk meets the big
 // occluders first, so its best t falls early and later boxes are culled
 // (1% on the Cornell box).  The order changes no hit.
-Status flat_build(uint32_t n, const DevBuf& nodes, const BvhScratch& s, DevBuf& flat, hipStream_t st) {
+Status flat_build(uint32_t n, const DevBuf& nodes, const BvhScratch& s, DevBuf& flat, hipStream_t st,
+                  float& overlap) {
+    overlap = 0.0f;
     if (n == 0 || n > kFlatMaxPrims) return Status::ok();
     AUR_TRY(flat.alloc((size_t)n * 32));
     k_flat_fill<<<blocks_for(n, kBlock), kBlock, 0, st>>>(n, s.leaf_pos.as<uint32_t>(), nodes.as<float4>(),
@@ -720,6 +722,19 @@ Status flat_build(uint32_t n, const DevBuf& nodes, const BvhScratch& s, DevBuf& 
     std::vector<uint32_t> idx(n);
     for (uint32_t i = 0; i < n; ++i) idx[i] = i;
     std::stable_sort(idx.begin(), idx.end(), [&](uint32_t a, uint32_t b) { return area(a) > area(b); });
+    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY}, sum = 0.0f;
+    for (uint32_t i = 0; i < n; ++i) {
+        const float4 l = rec[2 * (size_t)i], h = rec[2 * (size_t)i + 1];
+        lo[0] = std::min(lo[0], l.x);
+        lo[1] = std::min(lo[1], l.y);
+        lo[2] = std::min(lo[2], l.z);
+        hi[0] = std::max(hi[0], h.x);
+        hi[1] = std::max(hi[1], h.y);
+        hi[2] = std::max(hi[2], h.z);
+        sum += area(i);
+    }
+    const float dx = hi[0] - lo[0], dy = hi[1] - lo[1], dz = hi[2] - lo[2], all = dx * dy + dy * dz + dz * dx;
+    overlap = all > 0.0f ? sum / all : 0.0f;
     for (uint32_t i = 0; i < n; ++i) {
         sorted[2 * (size_t)i] = rec[2 * (size_t)idx[i]];
         sorted[2 * (size_t)i + 1] = rec[2 * (size_t)idx[i] + 1];

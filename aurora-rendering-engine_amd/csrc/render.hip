@@ -89,19 +89,29 @@ __device__ __forceinline__ void camera_ray(const CamF& cam, uint32_t pixel, uint
 
 // ONE (in every kernel below): the pass holds a single scene, so its record
 // is read at a wave-uniform address (scalar loads) instead of per path.
-template <bool ONE>
-__global__ __launch_bounds__(kBlock) void k_raygen(Pass pa, float4* qo, float4* qd, float4* qb, float4* L,
-                                                   uint32_t* counters) {
+// BYVAL (k_raygen): that record comes with the launch and block 0 writes it to
+// the table for the kernels that follow, so a pass needs no copy of its own
+// before it (a copy and its hand-over cost a small frame 10 us; a captured pass,
+// whose record advances on the device, reads the table).
+template <bool ONE, bool BYVAL>
+__global__ __launch_bounds__(kBlock) void k_raygen(Pass pa, SceneRec rec, SceneRec* table, float4* qo, float4* qd,
+                                                   float4* qb, float4* L, uint32_t* counters) {
     const uint32_t p = blockIdx.x * kBlock + threadIdx.x;
     const uint32_t n = pa.n_paths;
+    if constexpr (BYVAL) {
+        if (p == 0) *table = rec;
+    }
     if (p == 0) {
         counters[0] = n;   // queue 0 count
         counters[1] = 0u;  // queue 1 count (the segment counter spans the call)
+        if (pa.first) counters[kTailSegs] = counters[kTailSegs + 1] = 0u;
     }
-    if (p < kPools) counters[kPoolBase + kPoolStride * p] = 0u;  // extend work pools
+    if (p < kPools) counters[kPoolBase + kPoolStride * p] = 0u;  // work pools
     if (p >= n) return;
     const uint32_t sid = ONE ? 0u : find_rec<false>(pa.recs, pa.n_recs, p);
-    const SceneRec r = scene_rec<ONE>(pa.recs, sid);
+    SceneRec r;
+    if constexpr (BYVAL) r = rec;
+    else r = scene_rec<ONE>(pa.recs, sid);
     const uint32_t local = p - r.path_off;
     const uint32_t s_local = local / r.WH;
     const uint32_t pixel = local - s_local * r.WH;
@@ -585,11 +595,12 @@ ShadeBufs shade_bufs(Workspace& ws, int cur) {
 
 }  // namespace
 
-Status launch_raygen(const Pass& p, Workspace& ws, hipStream_t s) {
+Status launch_raygen(const Pass& p, const SceneRec* rec, Workspace& ws, hipStream_t s) {
     const uint32_t blocks = std::max<uint32_t>(1, (p.n_paths + kBlock - 1) / kBlock);
-    auto k = p.n_recs == 1 ? k_raygen<true> : k_raygen<false>;
-    k<<<blocks, kBlock, 0, s>>>(p, ws.q_o[0].as<float4>(), ws.q_d[0].as<float4>(), ws.q_b[0].as<float4>(),
-                                ws.L.as<float4>(), ws.counters.as<uint32_t>());
+    auto k = rec ? k_raygen<true, true> : p.n_recs == 1 ? k_raygen<true, false> : k_raygen<false, false>;
+    k<<<blocks, kBlock, 0, s>>>(p, rec ? *rec : SceneRec{}, ws.recs.as<SceneRec>(), ws.q_o[0].as<float4>(),
+                                ws.q_d[0].as<float4>(), ws.q_b[0].as<float4>(), ws.L.as<float4>(),
+                                ws.counters.as<uint32_t>());
     AUR_HIP(hipGetLastError());
     return Status::ok();
 }

@@ -242,8 +242,10 @@ int aurora_set_launch(aurora_ctx* ctx, int extend_blocks_per_cu,
 int aurora_set_queue(aurora_ctx* ctx, uint32_t pass_paths, uint32_t claim_paths);
 
 /* Tree walked by the render kernels: 0 = the binary LBVH (default; one
- * 64-byte child pair per step), 1 = the four-wide tree (one 128-byte node
- * per step), 2 = flat: for single-scene renders of scenes of at most 256
+ * 64-byte child pair per step; the persistent path kernel takes the flat form
+ * for a single scene of at most 64 primitives whose leaf boxes' areas add up to
+ * the scene box's, such as a small closed room), 1 = the four-wide tree (one
+ * 128-byte node per step), 2 = flat: for single-scene renders of scenes of at most 256
  * primitives, the persistent path kernel tests every leaf in Morton order,
  * the same sequence for every ray (no stack, no divergence); elsewhere 2
  * walks the four-wide tree.  Which is fastest depends on the scene (the
