@@ -75,21 +75,41 @@ struct EventPair {
     }
 };
 
+// What the host reads during a build (the per-depth node counts, then bounds and
+// counts) in pinned memory, and the build's events: kept, since creating them
+// and copying to pageable memory took 50 us per build.
+struct BvhHost {
+    uint32_t* p = nullptr;  // 257 words
+    EventPair ev;           // the build's timing
+    hipEvent_t starts = nullptr;
+    Status create() {
+        if (!ev.e[0]) AUR_TRY(ev.create());
+        if (!starts) AUR_HIP(hipEventCreateWithFlags(&starts, hipEventDisableTiming));
+        if (!p) AUR_HIP(hipHostMalloc((void**)&p, 257 * 4, hipHostMallocDefault));
+        return Status::ok();
+    }
+    ~BvhHost() {
+        if (starts) (void)hipEventDestroy(starts);
+        if (p) (void)hipHostFree(p);
+    }
+};
+
 // Scratch of the LBVH build.
 struct BvhScratch {
+    BvhHost host;
     DevBuf box_lo, box_hi;      // float4 per prim (padded boxes)
-    DevBuf bounds;              // 12 ordered-u32: scene lo/hi, centroid lo/hi
+    DevBuf bounds;              // 12 ordered-u32: scene lo/hi, centroid lo/hi; deepest wide level; wide nodes
     DevBuf bpart;               // 12 ordered-u32 per block of the bounds reduction
     DevBuf keys[2], vals[2];    // radix sort ping-pong
     DevBuf hist;                // 256 * blocks
     DevBuf gamma, flags, int_parent, leaf_parent, int_pos, leaf_pos;
-    DevBuf jump[2];             // (ancestor, distance) per internal node, pointer-jumping ping-pong
+    DevBuf cut;                 // four-wide cut of each internal node (uint4)
     DevBuf lvl_key, lvl_node;   // internal nodes sorted by depth
     DevBuf lvl_start;           // first sorted index of each depth (257 u32)
     DevBuf widx;                // wide index of each internal node (exclusive scan of even-depth flags)
     void release() {
         DevBuf* all[] = {&box_lo, &box_hi, &bounds, &bpart, &keys[0], &keys[1], &vals[0], &vals[1], &hist, &gamma,
-                         &flags, &int_parent, &leaf_parent, &int_pos, &leaf_pos, &jump[0], &jump[1], &lvl_key,
+                         &flags, &int_parent, &leaf_parent, &int_pos, &leaf_pos, &cut, &lvl_key,
                          &lvl_node, &lvl_start, &widx};
         for (DevBuf* b : all) b->release();
     }

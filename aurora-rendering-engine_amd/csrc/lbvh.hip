@@ -6,14 +6,15 @@
 //   -> k_morton (30-bit codes) -> 4 x {k_hist, scan, k_scatter} (stable LSD
 //   radix sort of (code, id) with 8-bit digits; the scatter ranks keys with
 //   wave64 ballots and LDS per-wave digit counts) -> k_karras (Karras 2012
-//   radix tree) -> depth of every internal node by pointer jumping
-//   (k_jump_init, 7 x k_jump, k_jump_out) -> internal nodes sorted by depth
-//   (one radix pass) -> k_leaves, then one k_refit_level per depth, deepest
-//   first -> four-wide tree: one k_wide_mark per depth, shallowest first, a
-//   scan of the wide-node flags, k_wide_fill.  Each level reads child boxes written by earlier launches, so the
-//   refit needs no arrival counters: on gfx950 an agent-scope acquire or
-//   release writes back or invalidates the XCD's L2, and one pair per node
-//   cost 19 ms at 4M primitives.
+//   radix tree) -> depth of every internal node (k_depth) -> internal nodes
+//   sorted by depth (one radix pass) -> k_leaves, then the refit by depth,
+//   deepest first -> four-wide tree: the cut of every internal node
+//   (k_wide_cut), the wide nodes marked by depth, shallowest first, a scan of
+//   their flags, k_wide_fill.  Runs of depths of few nodes share a launch.
+//   Each level reads child boxes written by earlier launches or, within such a
+//   run, by the same block, so the refit needs no arrival counters: on gfx950
+//   an agent-scope acquire or release writes back or invalidates the XCD's L2,
+//   and one pair per node cost 19 ms at 4M primitives.
 //
 // Layout: node 0 is the root, node 1 padding; the children of the internal
 // node with split gamma sit at 2+2*gamma and 3+2*gamma, so every child pair
@@ -280,6 +281,51 @@ __global__ __launch_bounds__(kBlock) void k_scan_apply(uint32_t* h, uint32_t tot
     }
 }
 
+// The same scan in one launch, out of place, for counts where reading all that
+// lies before a tile costs less than two more launches: each block of 1024
+// threads sums the entries before its 4096 itself, 16 bytes per thread and
+// trip, out of the L2.  50 K entries (400 K primitives' digit counts): 6 us
+// against 14 us for the three launches (and 46 us for one block walking them
+// all).  The line: at 256 K entries the last block makes 63 trips.
+constexpr uint32_t kScanOneMax = 262144;
+constexpr uint32_t kScanOneTile = 4096;
+__global__ __launch_bounds__(1024) void k_scan_one(const uint32_t* in, uint32_t* out, uint32_t total) {
+    __shared__ uint32_t red[16], pre[16];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint4* in4 = reinterpret_cast<const uint4*>(in);  // 16-byte aligned (scan_exclusive)
+    uint32_t p = 0;
+#pragma unroll 8
+    for (uint32_t b = 0; b < blockIdx.x; ++b) {
+        const uint4 v = in4[b * 1024u + tid];
+        p += v.x + v.y + v.z + v.w;
+    }
+    const uint32_t at = blockIdx.x * kScanOneTile + 4u * tid;
+    uint32_t v[4], sum = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+        v[j] = at + j < total ? in[at + j] : 0u;
+        sum += v[j];
+    }
+    uint32_t inc = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t u = __shfl_up(inc, o);
+        if ((int)lane >= o) inc += u;
+    }
+    for (int o = 32; o > 0; o >>= 1) p += __shfl_xor(p, o);
+    if (lane == 63) red[wave] = inc;
+    if (lane == 0) pre[wave] = p;
+    __syncthreads();
+    uint32_t run = inc - sum;
+#pragma unroll
+    for (uint32_t w = 0; w < 16; ++w) run += pre[w] + (w < wave ? red[w] : 0u);
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+        if (at + j < total) out[at + j] = run;
+        run += v[j];
+    }
+}
+
 // stable scatter: ranks within a wave from 8 ballots over the digit bits,
 // across the 4 waves of a 256-key chunk through LDS counts
 __global__ __launch_bounds__(kBlock) void k_scatter(const uint32_t* kin, const uint32_t* vin, uint32_t* kout,
@@ -408,14 +454,10 @@ __global__ __launch_bounds__(kBlock) void k_flat_fill(uint32_t n, const uint32_t
     flat[2 * (size_t)m + 1] = nodes[2 * pos + 1];
 }
 
-// the internal nodes of one depth: union of the two child records (written
-// by earlier launches), child index, parent position
-__global__ __launch_bounds__(kBlock) void k_refit_level(const uint32_t* lvl_node, uint32_t count,
-                                                        const uint32_t* gamma, const uint32_t* int_pos,
-                                                        const uint32_t* int_parent, float4* nodes) {
-    const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
-    if (k >= count) return;
-    const uint32_t i = lvl_node[k];
+// an internal node: union of the two child records (of deeper levels), child
+// index, parent position
+__device__ __forceinline__ void refit_node(uint32_t i, const uint32_t* gamma, const uint32_t* int_pos,
+                                           const uint32_t* int_parent, float4* nodes) {
     const uint32_t c = 2 + 2 * gamma[i];
     const float4 a0 = nodes[2 * (size_t)c], a1 = nodes[2 * (size_t)c + 1];
     const float4 b0 = nodes[2 * (size_t)c + 2], b1 = nodes[2 * (size_t)c + 3];
@@ -424,47 +466,48 @@ __global__ __launch_bounds__(kBlock) void k_refit_level(const uint32_t* lvl_node
     nodes[2 * (size_t)pos] = make_float4(fminf(a0.x, b0.x), fminf(a0.y, b0.y), fminf(a0.z, b0.z), __uint_as_float(c));
     nodes[2 * (size_t)pos + 1] = make_float4(fmaxf(a1.x, b1.x), fmaxf(a1.y, b1.y), fmaxf(a1.z, b1.z), __uint_as_float(gp));
 }
-
-// ---- depth of every internal node by pointer jumping ----
-// J[i] = (ancestor a of i, number of edges from i up to a); kNone marks the
-// root's parent.  A round replaces (a, d) by (ancestor of a, d + its
-// distance), doubling the span, so after r rounds every node within 2^r
-// edges of the root is resolved.  A Karras tree over distinct 64-bit keys
-// (30-bit code, 32-bit index) is at most 64 internal levels deep: each
-// child's common prefix is longer than its parent's.  Seven rounds cover 128.
-constexpr int kJumpRounds = 7;
-
-__global__ __launch_bounds__(kBlock) void k_jump_init(uint32_t ni, const uint32_t* int_parent, uint2* J) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= ni) return;
-    const uint32_t p = int_parent[i];
-    J[i] = make_uint2(p, p == kNone ? 0u : 1u);
+// the nodes of one depth
+__global__ __launch_bounds__(kBlock) void k_refit_level(const uint32_t* lvl_node, uint32_t count,
+                                                        const uint32_t* gamma, const uint32_t* int_pos,
+                                                        const uint32_t* int_parent, float4* nodes) {
+    const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+    if (k < count) refit_node(lvl_node[k], gamma, int_pos, int_parent, nodes);
 }
-
-__global__ __launch_bounds__(kBlock) void k_jump(uint32_t ni, const uint2* A, uint2* B) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= ni) return;
-    const uint2 a = A[i];
-    if (a.x == kNone) {
-        B[i] = a;
-        return;
+// Consecutive depths of at most kSmallLevel nodes each, by one block with a
+// barrier between them: the upper half of a tree's depths and its last ones
+// hold few nodes, and a launch of its own costs each 5 us.
+constexpr uint32_t kSmallLevel = 2048;
+__global__ __launch_bounds__(1024) void k_refit_levels(const uint32_t* lvl_node, const uint32_t* starts, int deepest,
+                                                       int top, const uint32_t* gamma, const uint32_t* int_pos,
+                                                       const uint32_t* int_parent, float4* nodes) {
+    for (int d = deepest; d >= top; --d) {
+        for (uint32_t k = starts[d] + threadIdx.x; k < starts[d + 1]; k += 1024)
+            refit_node(lvl_node[k], gamma, int_pos, int_parent, nodes);
+        __syncthreads();
     }
-    const uint2 q = A[a.x];
-    B[i] = make_uint2(q.x, a.y + q.y);
 }
 
-// depth keys for the level sort (255 marks a node left unresolved, which the
+// ---- depth of every internal node ----
+// Each node walks up to the root.  A Karras tree over distinct 64-bit keys
+// (30-bit code, 32-bit index) is at most 64 internal levels deep (each child's
+// common prefix is longer than its parent's), and the parents near the root stay
+// in cache: 400 K nodes take 10 us, where pointer jumping took nine launches and 44 us.
+// Depth keys for the level sort (255 marks a node left unresolved, which the
 // host reports), node ids, and the wide-node flags cleared but for the root
 // (k_wide_mark sets the others); flag[ni] = 0 so the exclusive scan leaves
 // the wide-node count at [ni]
-__global__ __launch_bounds__(kBlock) void k_jump_out(uint32_t ni, const uint2* J, uint32_t* key, uint32_t* id,
-                                                     uint32_t* wflag) {
+__global__ __launch_bounds__(kBlock) void k_depth(uint32_t ni, const uint32_t* int_parent, uint32_t* key, uint32_t* id,
+                                                  uint32_t* wflag, uint32_t* maxlv) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i > ni) return;
     wflag[i] = i == 0 && ni > 0 ? 1u : 0u;  // wide level of the root
+    if (i == 0) *maxlv = 0u;
     if (i == ni) return;
-    const uint2 a = J[i];
-    const uint32_t d = (a.x == kNone && a.y < 255u) ? a.y : 255u;
+    uint32_t d = 0, p = int_parent[i];
+    while (p != kNone && d < 255u) {
+        ++d;
+        p = int_parent[p];
+    }
     key[i] = d;
     id[i] = i;
 }
@@ -575,28 +618,55 @@ __device__ __forceinline__ int wide_cut(uint32_t i, const uint32_t* gamma, const
     return k;
 }
 
-// the flagged internal nodes of one depth flag the internal nodes of their
-// cuts with their own wide level plus one (the root's level is 1)
-__global__ __launch_bounds__(kBlock) void k_wide_mark(const uint32_t* lvl_node, uint32_t count,
-                                                      const uint32_t* gamma, const uint32_t* flags,
-                                                      const float4* nodes, bool greedy, uint32_t* wflag) {
-    const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
-    if (k >= count) return;
-    const uint32_t i = lvl_node[k];
-    const uint32_t lv = wflag[i];
-    if (!lv) return;
+// The cut of every internal node, whether it becomes a wide node or not: four
+// words of (internal index << 1) or (leaf's binary position << 1 | 1), kNone for
+// an unused slot.  The cut is a chain of dependent loads (6 us at the least);
+// taken here once for all nodes in parallel, it leaves the top-down marking one
+// load per level, and the fill none to repeat.
+__global__ __launch_bounds__(kBlock) void k_wide_cut(uint32_t ni, const uint32_t* gamma, const uint32_t* flags,
+                                                     const float4* nodes, bool greedy, uint4* cut) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= ni) return;
     WideRef r[4];
     const int m = wide_cut(i, gamma, flags, nodes, greedy, r);
-    for (int q = 0; q < m; ++q)
-        if (!r[q].leaf) wflag[r[q].j] = lv + 1u;
+    uint32_t w[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) w[q] = q >= m ? kNone : r[q].leaf ? (r[q].pos << 1) | 1u : r[q].j << 1;
+    cut[i] = make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// a flagged internal node flags the internal nodes of its cut with its own
+// wide level plus one (the root's level is 1)
+__device__ __forceinline__ void mark_node(uint32_t i, const uint4* cut, uint32_t* wflag) {
+    const uint32_t lv = wflag[i];
+    if (!lv) return;
+    const uint4 c = cut[i];
+    const uint32_t w[4] = {c.x, c.y, c.z, c.w};
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        if (!(w[q] & 1u)) wflag[w[q] >> 1] = lv + 1u;  // (kNone is odd)
+}
+// the internal nodes of one depth
+__global__ __launch_bounds__(kBlock) void k_wide_mark(const uint32_t* lvl_node, uint32_t count, const uint4* cut,
+                                                      uint32_t* wflag) {
+    const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+    if (k < count) mark_node(lvl_node[k], cut, wflag);
+}
+// consecutive depths of few nodes, as k_refit_levels
+__global__ __launch_bounds__(1024) void k_wide_marks(const uint32_t* lvl_node, const uint32_t* starts, int top,
+                                                     int deepest, const uint4* cut, uint32_t* wflag) {
+    for (int d = top; d <= deepest; ++d) {
+        for (uint32_t k = starts[d] + threadIdx.x; k < starts[d + 1]; k += 1024) mark_node(lvl_node[k], cut, wflag);
+        __syncthreads();
+    }
 }
 
 // the deepest wide level into *maxlv (0 before the launch), and the levels
 // turned into the 0/1 flags that the scan numbers.  Grid-stride over at
 // most kLevelsGrid blocks, reduced in the block: one atomic per block (one
 // per wave on a single address serialised 62 K atomics, 0.7 ms, on 4 M
-// primitives)
-constexpr uint32_t kLevelsGrid = 1024;
+// primitives, and 1024 blocks' 10 us of the 14 that 400 K nodes took)
+constexpr uint32_t kLevelsGrid = 256;
 __global__ __launch_bounds__(kBlock) void k_wide_levels(uint32_t n, uint32_t* wflag, uint32_t* maxlv) {
     __shared__ uint32_t wave_max[kBlock / 64];
     uint32_t lv = 0u;
@@ -634,21 +704,23 @@ __device__ __forceinline__ void wide_slot(float4* w, int k, const float4* nodes,
 
 // one wide node per flagged internal node i, at widx[i] (the exclusive scan
 // of the flags): the slots of its cut (a leaf slot refers to its primitive,
-// an internal one to that node's wide index); unused slots are empty
-__global__ __launch_bounds__(kBlock) void k_wide_fill(uint32_t ni, const uint32_t* gamma, const uint32_t* flags,
-                                                      const uint32_t* widx, const float4* nodes, bool greedy,
-                                                      float4* wide) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+// an internal one to that node's wide index); unused slots are empty.  Four
+// threads per node, one per slot; the wide-node count for the host
+__global__ __launch_bounds__(kBlock) void k_wide_fill(uint32_t ni, const uint32_t* int_pos,
+                                                      const uint32_t* widx, const float4* nodes, const uint4* cut,
+                                                      float4* wide, uint32_t* n_wide) {
+    const uint32_t t = blockIdx.x * kBlock + threadIdx.x, i = t >> 2, q = t & 3u;
+    if (t == 0) *n_wide = widx[ni];
     if (i >= ni || widx[i + 1] == widx[i]) return;
     float4* w = wide + 8 * (size_t)widx[i];
-    WideRef r[4];
-    const int m = wide_cut(i, gamma, flags, nodes, greedy, r);
-    for (int q = 0; q < m; ++q)
-        wide_slot(w, q, nodes, r[q].pos, r[q].leaf ? __float_as_uint(nodes[2 * (size_t)r[q].pos].w) : widx[r[q].j]);
-    for (int q = m; q < 4; ++q) {
+    const uint32_t c = reinterpret_cast<const uint32_t*>(cut + i)[q];
+    if (c == kNone) {
         w[q] = make_float4(0.0f, 0.0f, 0.0f, __uint_as_float(AURORA_BVH4_EMPTY));
         w[4 + q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        return;
     }
+    const uint32_t pos = (c & 1u) ? c >> 1 : int_pos[c >> 1];
+    wide_slot(w, (int)q, nodes, pos, (c & 1u) ? __float_as_uint(nodes[2 * (size_t)pos].w) : widx[c >> 1]);
 }
 
 // a single primitive: one wide node holding the leaf
@@ -668,31 +740,38 @@ inline uint32_t blocks_for(uint64_t n, uint32_t per) { return (uint32_t)((n + pe
 // histogram entries of a sort of n keys, and the tile sums of its scan after them
 inline uint32_t hist_entries(uint32_t n) { return 256u * blocks_for(n, kTile); }
 
-void scan_exclusive(uint32_t* h, uint32_t total, hipStream_t st) {
+uint32_t* scan_exclusive(uint32_t* h, uint32_t* out, uint32_t total, hipStream_t st) {
+    if (total <= kScanOneMax) {
+        k_scan_one<<<blocks_for(total, kScanOneTile), 1024, 0, st>>>(h, out, total);
+        return out;
+    }
     uint32_t* part = h + total;
     const uint32_t np = blocks_for(total, kScanTile);
     k_scan_reduce<<<np, kBlock, 0, st>>>(h, total, part);
     k_scan_parts<<<1, kBlock, 0, st>>>(part, np);
     k_scan_apply<<<np, kBlock, 0, st>>>(h, total, part);
+    return h;
 }
 
 }  // namespace
 
 size_t radix_hist_bytes(uint32_t n) {
     const uint32_t e = hist_entries(n);
-    return ((size_t)e + blocks_for(e, kScanTile)) * 4;
+    return ((size_t)e + std::max(blocks_for(e, kScanTile), std::min(e, kScanOneMax))) * 4;
 }
 
 Status radix_sort_pairs(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, uint32_t* hist, uint32_t n,
                         int passes, hipStream_t st) {
     if (n == 0) return Status::ok();
     const uint32_t nb = blocks_for(n, kTile);
+    // the counts: behind their scan where that is out of place
+    uint32_t* raw = 256u * nb <= kScanOneMax ? hist + 256u * nb : hist;
     uint32_t* ks[2] = {k0, k1};
     uint32_t* vs[2] = {v0, v1};
     for (int pass = 0; pass < passes; ++pass) {
         const int a = pass & 1, b = a ^ 1;
-        k_hist<<<nb, kBlock, 0, st>>>(ks[a], n, 8 * pass, hist, nb);
-        scan_exclusive(hist, 256u * nb, st);
+        k_hist<<<nb, kBlock, 0, st>>>(ks[a], n, 8 * pass, raw, nb);
+        scan_exclusive(raw, hist, 256u * nb, st);
         k_scatter<<<nb, kBlock, 0, st>>>(ks[a], vs[a], ks[b], vs[b], n, 8 * pass, hist, nb);
     }
     AUR_HIP(hipGetLastError());
@@ -754,7 +833,6 @@ Status lbvh_build(const DevScene& sc_in, uint32_t n, DevBuf& nodes, DevBuf& wide
         return Status::ok();
     }
     const uint32_t n_nodes = n == 1 ? 1u : 2u * n;
-    const uint32_t nb = blocks_for(n, kTile);
     const uint32_t nbound = std::min<uint32_t>(blocks_for(n, kBlock), kBoundBlocks);
     AUR_TRY(nodes.alloc((size_t)n_nodes * 32));
     AUR_TRY(s.box_lo.alloc((size_t)n * 16));
@@ -773,9 +851,8 @@ Status lbvh_build(const DevScene& sc_in, uint32_t n, DevBuf& nodes, DevBuf& wide
     AUR_TRY(s.int_pos.alloc(ni * 4));
     AUR_TRY(s.leaf_parent.alloc((size_t)n * 4));
     AUR_TRY(s.leaf_pos.alloc((size_t)n * 4));
-    AUR_TRY(s.jump[0].alloc(ni * 8));
-    AUR_TRY(s.jump[1].alloc(ni * 8));
-    AUR_TRY(s.lvl_key.alloc(ni * 4));
+    AUR_TRY(s.cut.alloc(ni * 16));
+    AUR_TRY(s.lvl_key.alloc((ni + 1) * 4));
     AUR_TRY(s.lvl_node.alloc(ni * 4));
     AUR_TRY(s.lvl_start.alloc(257 * 4));
     const uint32_t n_flags = (uint32_t)ni + 1;
@@ -784,9 +861,8 @@ Status lbvh_build(const DevScene& sc_in, uint32_t n, DevBuf& nodes, DevBuf& wide
     // (every internal node)
     AUR_TRY(wide.alloc(ni * 128));
 
-    EventPair ev;
-    AUR_TRY(ev.create());
-    hipEvent_t e0 = ev.e[0], e1 = ev.e[1];
+    AUR_TRY(s.host.create());
+    hipEvent_t e0 = s.host.ev.e[0], e1 = s.host.ev.e[1];
     AUR_HIP(hipEventRecord(e0, st));
     k_prim_bounds<<<nbound, kBlock, 0, st>>>(sc, n, s.box_lo.as<float4>(), s.box_hi.as<float4>(),
                                              s.bpart.as<uint32_t>());
@@ -794,15 +870,11 @@ Status lbvh_build(const DevScene& sc_in, uint32_t n, DevBuf& nodes, DevBuf& wide
     k_morton<<<blocks_for(n, kBlock), kBlock, 0, st>>>(n, s.box_lo.as<float4>(), s.box_hi.as<float4>(),
                                                        s.bounds.as<uint32_t>(), s.keys[0].as<uint32_t>(),
                                                        s.vals[0].as<uint32_t>());
-    for (int pass = 0; pass < 4; ++pass) {
-        const int a = pass & 1, b = a ^ 1;
-        k_hist<<<nb, kBlock, 0, st>>>(s.keys[a].as<uint32_t>(), n, 8 * pass, s.hist.as<uint32_t>(), nb);
-        scan_exclusive(s.hist.as<uint32_t>(), 256u * nb, st);
-        k_scatter<<<nb, kBlock, 0, st>>>(s.keys[a].as<uint32_t>(), s.vals[a].as<uint32_t>(), s.keys[b].as<uint32_t>(),
-                                         s.vals[b].as<uint32_t>(), n, 8 * pass, s.hist.as<uint32_t>(), nb);
-    }
+    AUR_TRY(radix_sort_pairs(s.keys[0].as<uint32_t>(), s.vals[0].as<uint32_t>(), s.keys[1].as<uint32_t>(),
+                             s.vals[1].as<uint32_t>(), s.hist.as<uint32_t>(), n, 4, st));
     // four passes: sorted data is back in buffer 0
     uint32_t depth = 0, n_wide = 1, wide_depth = 1;
+    uint32_t* const maxlv = s.bounds.as<uint32_t>() + 12;  // deepest wide level, then the wide-node count
     bool wide_greedy = false;
     if (n > 1) {
         const uint32_t nint = n - 1;
@@ -810,35 +882,44 @@ Status lbvh_build(const DevScene& sc_in, uint32_t n, DevBuf& nodes, DevBuf& wide
         k_karras<<<gi, kBlock, 0, st>>>(s.keys[0].as<uint32_t>(), n, s.gamma.as<uint32_t>(), s.flags.as<uint32_t>(),
                                         s.int_parent.as<uint32_t>(), s.leaf_parent.as<uint32_t>(),
                                         s.int_pos.as<uint32_t>(), s.leaf_pos.as<uint32_t>(), nodes.as<float4>());
-        uint2* J[2] = {s.jump[0].as<uint2>(), s.jump[1].as<uint2>()};
-        k_jump_init<<<gi, kBlock, 0, st>>>(nint, s.int_parent.as<uint32_t>(), J[0]);
-        for (int r = 0; r < kJumpRounds; ++r) k_jump<<<gi, kBlock, 0, st>>>(nint, J[r & 1], J[(r + 1) & 1]);
-        k_jump_out<<<blocks_for(nint + 1, kBlock), kBlock, 0, st>>>(nint, J[kJumpRounds & 1],
-                                                                    s.keys[1].as<uint32_t>(),
-                                                                    s.vals[1].as<uint32_t>(), s.widx.as<uint32_t>());
+        k_depth<<<blocks_for(nint + 1, kBlock), kBlock, 0, st>>>(nint, s.int_parent.as<uint32_t>(),
+                                                                 s.keys[1].as<uint32_t>(), s.vals[1].as<uint32_t>(),
+                                                                 s.widx.as<uint32_t>(), maxlv);
         // one 8-bit pass: the sorted pairs land in (lvl_key, lvl_node)
         AUR_TRY(radix_sort_pairs(s.keys[1].as<uint32_t>(), s.vals[1].as<uint32_t>(), s.lvl_key.as<uint32_t>(),
                                  s.lvl_node.as<uint32_t>(), s.hist.as<uint32_t>(), nint, 1, st));
         k_level_starts<<<1, 256, 0, st>>>(s.hist.as<uint32_t>(), blocks_for(nint, kTile), nint,
                                           s.lvl_start.as<uint32_t>());
-        uint32_t starts[257];
-        AUR_HIP(hipMemcpyAsync(starts, s.lvl_start.p, sizeof(starts), hipMemcpyDeviceToHost, st));
-        AUR_HIP(hipStreamSynchronize(st));
+        uint32_t* starts = s.host.p;
+        AUR_HIP(hipMemcpyAsync(starts, s.lvl_start.p, 257 * 4, hipMemcpyDeviceToHost, st));
+        AUR_HIP(hipEventRecord(s.host.starts, st));
+        // the leaf records need no depths: they are written while the host reads these
+        k_leaves<<<blocks_for(n, kBlock), kBlock, 0, st>>>(n, s.vals[0].as<uint32_t>(), s.box_lo.as<float4>(),
+                                                           s.box_hi.as<float4>(), s.leaf_pos.as<uint32_t>(),
+                                                           s.leaf_parent.as<uint32_t>(), s.int_pos.as<uint32_t>(),
+                                                           nodes.as<float4>());
+        AUR_HIP(hipEventSynchronize(s.host.starts));
         if (starts[255] != nint) return Status{AURORA_ERR_RUNTIME, "LBVH build: node depths did not resolve"};
         uint32_t maxd = 0;
         for (uint32_t d = 0; d < 255; ++d)
             if (starts[d + 1] > starts[d]) maxd = d;
         depth = maxd + 1;  // a deepest internal node has two leaf children
-        k_leaves<<<blocks_for(n, kBlock), kBlock, 0, st>>>(n, s.vals[0].as<uint32_t>(), s.box_lo.as<float4>(),
-                                                           s.box_hi.as<float4>(), s.leaf_pos.as<uint32_t>(),
-                                                           s.leaf_parent.as<uint32_t>(), s.int_pos.as<uint32_t>(),
-                                                           nodes.as<float4>());
-        for (int d = (int)maxd; d >= 0; --d) {
-            const uint32_t cnt = starts[d + 1] - starts[d];
-            if (cnt == 0) continue;
-            k_refit_level<<<blocks_for(cnt, kBlock), kBlock, 0, st>>>(
-                s.lvl_node.as<uint32_t>() + starts[d], cnt, s.gamma.as<uint32_t>(), s.int_pos.as<uint32_t>(),
-                s.int_parent.as<uint32_t>(), nodes.as<float4>());
+        // runs of levels of at most kSmallLevel nodes in one launch
+        auto small = [&](int d) { return starts[d + 1] - starts[d] <= kSmallLevel; };
+        for (int d = (int)maxd; d >= 0;) {
+            int top = d;
+            if (small(d)) {
+                while (top > 0 && small(top - 1)) --top;
+                k_refit_levels<<<1, 1024, 0, st>>>(s.lvl_node.as<uint32_t>(), s.lvl_start.as<uint32_t>(), d, top,
+                                                   s.gamma.as<uint32_t>(), s.int_pos.as<uint32_t>(),
+                                                   s.int_parent.as<uint32_t>(), nodes.as<float4>());
+            } else {
+                const uint32_t cnt = starts[d + 1] - starts[d];
+                k_refit_level<<<blocks_for(cnt, kBlock), kBlock, 0, st>>>(
+                    s.lvl_node.as<uint32_t>() + starts[d], cnt, s.gamma.as<uint32_t>(), s.int_pos.as<uint32_t>(),
+                    s.int_parent.as<uint32_t>(), nodes.as<float4>());
+            }
+            d = top - 1;
         }
         // four-wide traversal tree: levels top down, then the flags' scan and
         // the fill.  The walk pushes at most three nodes per wide level above
@@ -848,19 +929,29 @@ Status lbvh_build(const DevScene& sc_in, uint32_t n, DevBuf& nodes, DevBuf& wide
         if (depth > (uint32_t)kTravMaxStack)
             return Status{AURORA_ERR_RUNTIME, "LBVH build: tree deeper than the traversal stack"};
         bool greedy = n >= kWideGreedyMin;
-        uint32_t* maxlv = s.bounds.as<uint32_t>() + 12;
         for (int attempt = 0; attempt < 2; ++attempt) {
-            k_wide_reset<<<blocks_for(nint + 1, kBlock), kBlock, 0, st>>>(nint + 1, s.widx.as<uint32_t>(), maxlv);
-            for (uint32_t d = 0; d <= maxd; ++d) {
-                const uint32_t cnt = starts[d + 1] - starts[d];
-                if (cnt == 0) continue;
-                k_wide_mark<<<blocks_for(cnt, kBlock), kBlock, 0, st>>>(s.lvl_node.as<uint32_t>() + starts[d], cnt,
-                                                                         s.gamma.as<uint32_t>(),
-                                                                         s.flags.as<uint32_t>(), nodes.as<float4>(),
-                                                                         greedy, s.widx.as<uint32_t>());
+            if (attempt)
+                k_wide_reset<<<blocks_for(nint + 1, kBlock), kBlock, 0, st>>>(nint + 1, s.widx.as<uint32_t>(), maxlv);
+            k_wide_cut<<<gi, kBlock, 0, st>>>(nint, s.gamma.as<uint32_t>(), s.flags.as<uint32_t>(),
+                                              nodes.as<float4>(), greedy, s.cut.as<uint4>());
+            for (int d = 0; d <= (int)maxd;) {
+                int end = d;
+                if (small(d)) {
+                    while (end < (int)maxd && small(end + 1)) ++end;
+                    k_wide_marks<<<1, 1024, 0, st>>>(s.lvl_node.as<uint32_t>(), s.lvl_start.as<uint32_t>(), d, end,
+                                                     s.cut.as<uint4>(), s.widx.as<uint32_t>());
+                } else {
+                    const uint32_t cnt = starts[d + 1] - starts[d];
+                    k_wide_mark<<<blocks_for(cnt, kBlock), kBlock, 0, st>>>(s.lvl_node.as<uint32_t>() + starts[d], cnt,
+                                                                             s.cut.as<uint4>(), s.widx.as<uint32_t>());
+                }
+                d = end + 1;
             }
             k_wide_levels<<<std::min<uint32_t>(blocks_for(nint + 1, kBlock), kLevelsGrid), kBlock, 0, st>>>(
                 nint + 1, s.widx.as<uint32_t>(), maxlv);
+            // a wide level is at least one binary level: the host reads the
+            // deepest one only where the binary depth leaves a doubt
+            if (3u * (depth - 1u) <= (uint32_t)kTravMaxStack) break;
             AUR_HIP(hipMemcpyAsync(&wide_depth, maxlv, 4, hipMemcpyDeviceToHost, st));
             AUR_HIP(hipStreamSynchronize(st));
             if (3u * (wide_depth - 1u) <= (uint32_t)kTravMaxStack) break;
@@ -868,9 +959,11 @@ Status lbvh_build(const DevScene& sc_in, uint32_t n, DevBuf& nodes, DevBuf& wide
             greedy = false;
         }
         wide_greedy = greedy;
-        scan_exclusive(s.widx.as<uint32_t>(), nint + 1, st);
-        k_wide_fill<<<gi, kBlock, 0, st>>>(nint, s.gamma.as<uint32_t>(), s.flags.as<uint32_t>(),
-                                           s.widx.as<uint32_t>(), nodes.as<float4>(), greedy, wide.as<float4>());
+        // (the depth keys are read no more)
+        const uint32_t* wscan = scan_exclusive(s.widx.as<uint32_t>(), s.lvl_key.as<uint32_t>(), nint + 1, st);
+        k_wide_fill<<<blocks_for(4 * (uint64_t)nint, kBlock), kBlock, 0, st>>>(
+            nint, s.int_pos.as<uint32_t>(), wscan, nodes.as<float4>(), s.cut.as<uint4>(),
+            wide.as<float4>(), maxlv + 1);
     } else {
         k_leaves<<<1, kBlock, 0, st>>>(n, s.vals[0].as<uint32_t>(), s.box_lo.as<float4>(), s.box_hi.as<float4>(),
                                        s.leaf_pos.as<uint32_t>(), s.leaf_parent.as<uint32_t>(),
@@ -882,10 +975,13 @@ Status lbvh_build(const DevScene& sc_in, uint32_t n, DevBuf& nodes, DevBuf& wide
     std::swap(morton, s.keys[0]);
     std::swap(order, s.vals[0]);
 
-    uint32_t b[12];
-    AUR_HIP(hipMemcpyAsync(b, s.bounds.p, 48, hipMemcpyDeviceToHost, st));
-    if (n > 1) AUR_HIP(hipMemcpyAsync(&n_wide, s.widx.as<uint32_t>() + (n - 1), 4, hipMemcpyDeviceToHost, st));
+    uint32_t* b = s.host.p;
+    AUR_HIP(hipMemcpyAsync(b, s.bounds.p, 14 * 4, hipMemcpyDeviceToHost, st));
     AUR_HIP(hipStreamSynchronize(st));
+    if (n > 1) {
+        wide_depth = b[12];
+        n_wide = b[13];
+    }
     float ms = 0.0f;
     AUR_HIP(hipEventElapsedTime(&ms, e0, e1));
     local.n_nodes = n_nodes;
