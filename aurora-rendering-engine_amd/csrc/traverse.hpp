@@ -1,10 +1,11 @@
-// traverse.hpp — closest-hit traversal over the LBVH, in two forms.
+// traverse.hpp — closest-hit traversal over the LBVH: one lane per ray over the
+// binary or the four-wide tree, and four lanes per ray over the four-wide tree
+// (the group walk, below; uncounted queries and bounces of large scenes).
 // Four-wide: the 128-byte node (one cache line) holds four child boxes; per
 // step the four slab tests against the current best t, the hit leaf
 // primitives in slot order, then descend to the nearest hit internal slot
 // and push the others farthest first.  It halves the dependent fetches and
-// uses whole lines, so it wins where traversal is memory bound (large
-// incoherent ray queries).  Binary: the 64-byte child pair per step, a
+// uses whole lines, so it wins where traversal is memory bound.  Binary: the 64-byte child pair per step, a
 // cheaper step that wins where traversal is issue bound (render bounces,
 // whose nodes sit in cache).
 //
