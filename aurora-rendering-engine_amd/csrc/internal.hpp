@@ -266,10 +266,13 @@ struct PatchWork {
 Status patch_check(const aurora_patch_triangle* tris, uint32_t n_tris, const aurora_patch_material* mats,
                    uint32_t n_mats, const aurora_patch_camera* cam, const aurora_patch_config* cfg);
 // plan on the host, rasterise on stream s into d_out (H x W x 3 doubles);
-// returns after the raster launches completed (stats->kernel_ms)
+// returns after the raster launches completed (stats->kernel_ms).  A frame of
+// more than max_textures textures is refused, with the plan's size in stats.
+constexpr uint32_t kPatchMaxTextures = 1u << 26;
 Status patch_render_device(PatchWork& pw, const aurora_patch_triangle* tris, uint32_t n_tris,
                            const aurora_patch_material* mats, const aurora_patch_camera* cam,
-                           const aurora_patch_config* cfg, double* d_out, hipStream_t s, aurora_patch_stats* stats);
+                           const aurora_patch_config* cfg, double* d_out, hipStream_t s, aurora_patch_stats* stats,
+                           uint32_t max_textures = kPatchMaxTextures);
 // 8-bit resolve of n floats (sum and out 16-byte and 4-byte aligned)
 Status launch_resolve_rgb8(const float* sum, size_t n, uint32_t spp, uint32_t transfer, uint8_t* out, hipStream_t s);
 Status launch_shade(const Pass& p, Workspace& ws, int cur, uint32_t depth, int grid, hipStream_t s);

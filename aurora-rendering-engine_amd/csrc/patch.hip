@@ -215,6 +215,8 @@ struct PatchTile {
 };
 
 // ---- planner -------------------------------------------------------------
+Status too_many_textures() { return Status{AURORA_ERR_NOMEM, "patch render: recursion tree above 2^26 textures"}; }
+
 struct Plan {
     const std::vector<HTri>* scene = nullptr;
     const Verts* verts = nullptr;
@@ -232,10 +234,11 @@ struct Plan {
     };
     std::vector<Level> levels;
     // empty tables that keep their storage
-    void reset(const std::vector<HTri>& sc, const Verts& v, const aurora_patch_config& c) {
+    void reset(const std::vector<HTri>& sc, const Verts& v, const aurora_patch_config& c, uint32_t limit) {
         scene = &sc;
         verts = &v;
         cfg = c;
+        max_textures = limit;
         texs.clear();
         tex_depth.clear();
         warps.clear();
@@ -248,6 +251,7 @@ struct Plan {
     std::vector<int> tex_depth;
     std::vector<PatchWarp> warps;
     size_t tex_base = 0;  // the first texture of the subtree at work
+    uint32_t max_textures = kPatchMaxTextures;
     uint64_t pool_texels = 0;
     uint64_t warp_texels = 0;
     int max_level = -1;
@@ -381,8 +385,8 @@ struct Plan {
         tw = clampi(tw, cfg.min_tex_res, cfg.max_tex_res);
         th = clampi(th, cfg.min_tex_res, cfg.max_tex_res);
         const uint32_t idx = uint32_t(texs.size());
-        if (texs.size() - tex_base >= (1u << 26)) {
-            status = Status{AURORA_ERR_NOMEM, "patch render: recursion tree above 2^26 textures"};
+        if (texs.size() - tex_base >= max_textures) {
+            status = too_many_textures();
             return idx;
         }
         PatchTex T{};
@@ -458,9 +462,10 @@ struct FramePlan {
     }
 };
 
+// max_textures: the most of the whole frame (and of one subtree);
 // max_threads 0: the library's choice
 Status plan_frame(std::vector<HTri>& scene, const aurora_patch_config& cfg, P3 eye, const HTri vp[2], int W,
-                  int H, FramePlan& out, unsigned max_threads = 0) {
+                  int H, uint32_t max_textures, FramePlan& out, unsigned max_threads = 0) {
     // distinct vertex positions (bitwise), in first-seen order
     Verts verts;
     {
@@ -499,7 +504,7 @@ Status plan_frame(std::vector<HTri>& scene, const aurora_patch_config& cfg, P3 e
         double px;
         Poly poly;
     };
-    for (Plan& p : out.worker) p.reset(scene, verts, cfg);
+    for (Plan& p : out.worker) p.reset(scene, verts, cfg, max_textures);
     Plan& top = out.worker[0];
     std::vector<Top> items;
     Poly poly;
@@ -515,13 +520,16 @@ Status plan_frame(std::vector<HTri>& scene, const aurora_patch_config& cfg, P3 e
     struct Span {
         const Plan* by;
         size_t tex0, tex1, warp0, warp1;
-        uint64_t pool0, pool1;
+        uint64_t pool0, pool1, warp_texels;
+        int max_level;
     };
     std::vector<Span> span(items.size());
     auto run = [&](size_t i, Plan& p) {
         Span& a = span[i];
-        a = Span{&p, p.texs.size(), 0, p.warps.size(), 0, p.pool_texels, 0};
+        a = Span{&p, p.texs.size(), 0, p.warps.size(), 0, p.pool_texels, 0, 0, -1};
         p.tex_base = a.tex0;
+        p.warp_texels = 0;
+        p.max_level = -1;
         p.path.clear();
         try {
             p.texture(eye, *items[i].tri, items[i].res, items[i].res, 0, items[i].px);
@@ -531,6 +539,8 @@ Status plan_frame(std::vector<HTri>& scene, const aurora_patch_config& cfg, P3 e
         a.tex1 = p.texs.size();
         a.warp1 = p.warps.size();
         a.pool1 = p.pool_texels;
+        a.warp_texels = p.warp_texels;
+        a.max_level = p.max_level;
     };
     const size_t work = items.size() * scene.size();
     const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
@@ -564,6 +574,7 @@ Status plan_frame(std::vector<HTri>& scene, const aurora_patch_config& cfg, P3 e
     out.tex_depth.reserve(n_texs);
     out.warps.reserve(n_warps + 2 * items.size() * 8);  // and the viewports' fans
     std::vector<uint32_t> root(items.size());
+    top.warp_texels = 0;  // (add_fan's below)
     for (int k = 0; k < 2; ++k) {
         for (size_t i = 0; i < items.size(); ++i) {
             if (items[i].vp != k) continue;
@@ -586,9 +597,12 @@ Status plan_frame(std::vector<HTri>& scene, const aurora_patch_config& cfg, P3 e
             out.tex_depth.insert(out.tex_depth.end(), p.tex_depth.begin() + long(a.tex0),
                                  p.tex_depth.begin() + long(a.tex1));
             out.pool_texels += a.pool1 - a.pool0;
+            out.warp_texels += a.warp_texels;
+            // raised with the textures themselves: a caller sizes its tables by
+            // it, also where the frame is refused here
+            out.max_level = std::max(out.max_level, a.max_level);
             root[i] = tex_off;
-            if (out.texs.size() > (1u << 26))
-                return Status{AURORA_ERR_NOMEM, "patch render: recursion tree above 2^26 textures"};
+            if (out.texs.size() > max_textures) return too_many_textures();
         }
         std::vector<PatchWarp> fans;
         for (size_t i = 0; i < items.size(); ++i)
@@ -597,10 +611,7 @@ Status plan_frame(std::vector<HTri>& scene, const aurora_patch_config& cfg, P3 e
         out.warps.insert(out.warps.end(), fans.begin(), fans.end());
         out.end[k] = uint32_t(out.warps.size());
     }
-    for (const Plan& p : out.worker) {
-        out.warp_texels += p.warp_texels;
-        out.max_level = std::max(out.max_level, p.max_level);
-    }
+    out.warp_texels += top.warp_texels;
     return Status::ok();
 }
 
@@ -794,7 +805,8 @@ Status patch_check(const aurora_patch_triangle* tris, uint32_t n_tris, const aur
 
 Status patch_render_device(PatchWork& pw, const aurora_patch_triangle* tris, uint32_t n_tris,
                            const aurora_patch_material* mats, const aurora_patch_camera* cam,
-                           const aurora_patch_config* cfg, double* d_out, hipStream_t s, aurora_patch_stats* st) {
+                           const aurora_patch_config* cfg, double* d_out, hipStream_t s, aurora_patch_stats* st,
+                           uint32_t max_textures) {
     const auto t0 = std::chrono::steady_clock::now();
     std::vector<HTri> scene;
     scene.reserve(n_tris);
@@ -805,7 +817,7 @@ Status patch_render_device(PatchWork& pw, const aurora_patch_triangle* tris, uin
     // one plan per calling thread, kept between frames (see reset)
     static thread_local FramePlan plan;
     plan.reset();
-    const Status planned = plan_frame(scene, *cfg, eye, vps, W, H, plan);
+    const Status planned = plan_frame(scene, *cfg, eye, vps, W, H, max_textures, plan);
     RootArgs ra{};
     for (int k = 0; k < 2; ++k) {
         ra.begin[k] = plan.begin[k];
@@ -832,6 +844,21 @@ Status patch_render_device(PatchWork& pw, const aurora_patch_triangle* tris, uin
         texels += uint64_t(T.w) * T.h;
         level_off[size_t(plan.tex_depth[i]) + 1] += size_t(tiles_of(T.w)) * tiles_of(T.h);
     }
+    auto plan_stats = [&] {
+        if (!st) return;
+        st->textures = uint32_t(plan.texs.size());
+        st->raster_textures = raster;
+        st->levels = uint32_t(std::max(levels, 0));
+        st->warps = uint32_t(plan.warps.size());
+        st->texels = texels;
+        st->warp_texels = plan.warp_texels;
+        st->plan_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+        st->kernel_ms = 0.0;
+    };
+    if (planned.bad()) {
+        plan_stats();
+        return planned;
+    }
     for (int l = 0; l < levels; ++l) level_off[size_t(l) + 1] += level_off[size_t(l)];
     std::vector<PatchTile> tiles(levels > 0 ? level_off.back() : 0);
     std::vector<size_t> at(level_off);
@@ -844,18 +871,7 @@ Status patch_render_device(PatchWork& pw, const aurora_patch_triangle* tris, uin
             for (uint32_t tx = 0; tx < nx; ++tx) *t++ = PatchTile{uint32_t(i), uint16_t(tx), uint16_t(ty)};
         at[size_t(plan.tex_depth[i])] += size_t(nx) * ny;
     }
-    const auto t1 = std::chrono::steady_clock::now();
-    if (st) {
-        st->textures = uint32_t(plan.texs.size());
-        st->raster_textures = raster;
-        st->levels = uint32_t(std::max(levels, 0));
-        st->warps = uint32_t(plan.warps.size());
-        st->texels = texels;
-        st->warp_texels = plan.warp_texels;
-        st->plan_ms = std::chrono::duration<double, std::milli>(t1 - t0).count();
-        st->kernel_ms = 0.0;
-    }
-    AUR_TRY(planned);
+    plan_stats();
 
     AUR_TRY(pw.texs.alloc(std::max<size_t>(plan.texs.size(), 1) * sizeof(PatchTex)));
     AUR_TRY(pw.warps.alloc(std::max<size_t>(plan.warps.size(), 1) * sizeof(PatchWarp)));

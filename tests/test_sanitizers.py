@@ -3,7 +3,9 @@ checkpoints) under AddressSanitizer and UndefinedBehaviorSanitizer: g++
 builds oracle/san/san_main.cpp with them, which calls every oracle entry
 point on scenes of every primitive, material and texture kind (pairwise and
 greedy four-wide trees), the error paths, and feeds truncated and damaged
-files to the loaders.  Any report aborts the run (-fno-sanitize-recover)."""
+files to the loaders.  Any report aborts the run (-fno-sanitize-recover).
+The patch renderer's host code (csrc/patch.hip under hipcc's AddressSanitizer)
+refuses frames of too many textures, with the limit as a parameter."""
 import os
 import shutil
 import subprocess
@@ -24,3 +26,18 @@ def test_oracle_and_formats_are_clean_under_asan_and_ubsan(tmp_path):
     assert r.returncode == 0, (r.stdout + r.stderr)[-4000:]
     assert "san: ok" in r.stdout
     assert "runtime error" not in r.stderr and "AddressSanitizer" not in r.stderr
+
+
+@pytest.mark.skipif(not os.path.isdir(SAN) or not (shutil.which("hipcc") or os.path.exists("/opt/rocm/bin/hipcc")),
+                    reason="needs oracle/san and hipcc")
+def test_patch_frames_above_the_texture_limit_are_refused_clean_under_asan():
+    """Every subtree below the limit and their sum above it: AURORA_ERR_NOMEM,
+    the plan's size in the stats, and no access outside the tables."""
+    b = subprocess.run(["make", "-s", "-C", SAN, "../build/patch_limit"], capture_output=True, text=True, timeout=600)
+    assert b.returncode == 0, b.stderr[-3000:]
+    # (leaks: the HIP runtime's own, loaded with the library code)
+    env = dict(os.environ, ASAN_OPTIONS="detect_leaks=0:abort_on_error=0")
+    r = subprocess.run([os.path.join(ROOT, "oracle", "build", "patch_limit")], capture_output=True, text=True,
+                       timeout=600, env=env)
+    assert r.returncode == 0, (r.stdout + r.stderr)[-4000:]
+    assert "patch limit: ok" in r.stdout and "AddressSanitizer" not in r.stderr
