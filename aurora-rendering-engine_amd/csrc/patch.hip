@@ -215,6 +215,8 @@ struct PatchTile {
 };
 
 // ---- planner -------------------------------------------------------------
+template <class T> size_t held(const std::vector<T>& v) { return v.capacity() * sizeof(T); }
+
 Status too_many_textures() { return Status{AURORA_ERR_NOMEM, "patch render: recursion tree above 2^26 textures"}; }
 
 struct Plan {
@@ -233,6 +235,12 @@ struct Plan {
         std::vector<PatchWarp> mine;
     };
     std::vector<Level> levels;
+    size_t bytes() const {
+        size_t n = held(texs) + held(tex_depth) + held(warps);
+        for (const Level& l : levels)
+            n += held(l.proj.u) + held(l.proj.v) + held(l.proj.s) + held(l.seen) + held(l.mine);
+        return n;
+    }
     // empty tables that keep their storage
     void reset(const std::vector<HTri>& sc, const Verts& v, const aurora_patch_config& c, uint32_t limit) {
         scene = &sc;
@@ -442,6 +450,11 @@ struct Plan {
 // into its own tables, and merged in the serial order: texture, warp and
 // texel numbering equal a serial plan's.
 constexpr size_t kPlanThreads = 8;
+// What a calling thread keeps of a frame's tables for the next frame, at most:
+// per worker (of the 9,482 textures of a 1920x1080 mirror hall the largest holds
+// about 1 MB), and of the merged tables (3 MB there).  Larger tables are given
+// back when the frame is done.
+constexpr size_t kKeepWorkerBytes = 8u << 20, kKeepFrameBytes = 256u << 20;
 struct FramePlan {
     Plan worker[kPlanThreads];
     std::vector<PatchTex> texs;
@@ -460,7 +473,22 @@ struct FramePlan {
         pool_texels = warp_texels = 0;
         max_level = -1;
     }
+    size_t bytes() const { return held(texs) + held(tex_depth) + held(warps); }
+    void trim() {
+        for (Plan& p : worker)
+            if (p.bytes() > kKeepWorkerBytes) p = Plan();
+        if (bytes() > kKeepFrameBytes) {
+            std::vector<PatchTex>().swap(texs);
+            std::vector<int>().swap(tex_depth);
+            std::vector<PatchWarp>().swap(warps);
+        }
+    }
 };
+// one per calling thread, kept between frames (see reset)
+FramePlan& thread_plan() {
+    static thread_local FramePlan plan;
+    return plan;
+}
 
 // max_textures: the most of the whole frame (and of one subtree);
 // max_threads 0: the library's choice
@@ -814,9 +842,12 @@ Status patch_render_device(PatchWork& pw, const aurora_patch_triangle* tris, uin
     const P3 eye{cam->origin[0], cam->origin[1], cam->origin[2]};
     const int W = int(cam->width), H = int(cam->height);
     const HTri vps[2] = {host_tri(cam->viewport[0], nullptr), host_tri(cam->viewport[1], nullptr)};
-    // one plan per calling thread, kept between frames (see reset)
-    static thread_local FramePlan plan;
+    FramePlan& plan = thread_plan();
     plan.reset();
+    struct Trim {
+        FramePlan& p;
+        ~Trim() { p.trim(); }  // (after the copies to the device: the raster launches are waited for)
+    } trim{plan};
     const Status planned = plan_frame(scene, *cfg, eye, vps, W, H, max_textures, plan);
     RootArgs ra{};
     for (int k = 0; k < 2; ++k) {

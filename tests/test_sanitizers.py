@@ -5,7 +5,8 @@ point on scenes of every primitive, material and texture kind (pairwise and
 greedy four-wide trees), the error paths, and feeds truncated and damaged
 files to the loaders.  Any report aborts the run (-fno-sanitize-recover).
 The patch renderer's host code (csrc/patch.hip under hipcc's AddressSanitizer)
-refuses frames of too many textures, with the limit as a parameter."""
+refuses frames of too many textures, with the limit as a parameter, and keeps no
+more than its stated sizes of a large frame's tables."""
 import os
 import shutil
 import subprocess
@@ -30,9 +31,10 @@ def test_oracle_and_formats_are_clean_under_asan_and_ubsan(tmp_path):
 
 @pytest.mark.skipif(not os.path.isdir(SAN) or not (shutil.which("hipcc") or os.path.exists("/opt/rocm/bin/hipcc")),
                     reason="needs oracle/san and hipcc")
-def test_patch_frames_above_the_texture_limit_are_refused_clean_under_asan():
+def test_patch_tables_stay_in_their_limits_under_asan():
     """Every subtree below the limit and their sum above it: AURORA_ERR_NOMEM,
-    the plan's size in the stats, and no access outside the tables."""
+    the plan's size in the stats, and no access outside the tables.  After a large
+    frame the thread keeps at most the stated sizes."""
     b = subprocess.run(["make", "-s", "-C", SAN, "../build/patch_limit"], capture_output=True, text=True, timeout=600)
     assert b.returncode == 0, b.stderr[-3000:]
     # (leaks: the HIP runtime's own, loaded with the library code)
