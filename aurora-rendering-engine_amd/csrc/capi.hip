@@ -59,6 +59,7 @@ struct aurora_ctx {
     hipEvent_t recs_ev[2] = {nullptr, nullptr};
     int recs_turn = 0;
     std::vector<hipEvent_t> cnt_ev;  // wavefront bounces: their live-path counts have arrived
+    BvhHost bvh_host;                // the LBVH builds' pinned words and events
     uint32_t host_recs_cap = 0;
     unsigned char* scratch = nullptr;  // this device's copy of the allocation-free scratch array
     PatchWork patch;                   // patch-projection renderer tables
@@ -1178,7 +1179,7 @@ int aurora_bvh_build(aurora_scene* s, aurora_bvh_stats* stats) {
     aurora_ctx* c = s->ctx;
     CK(c, hip_status(hipSetDevice(c->device), "hipSetDevice"));
     aurora_bvh_stats st{};
-    CK(c, lbvh_build(s->view, s->n_prims, s->nodes, s->wide, s->morton, s->order, s->scr, c->stream, &st));
+    CK(c, lbvh_build(s->view, s->n_prims, s->nodes, s->wide, s->morton, s->order, s->scr, c->bvh_host, c->stream, &st));
     s->view.nodes = s->nodes.as<float4>();
     s->view.n_nodes = st.n_nodes;
     s->view.wide = s->wide.as<float4>();

@@ -76,8 +76,10 @@ struct EventPair {
 };
 
 // What the host reads during a build (the per-depth node counts, then bounds and
-// counts) in pinned memory, and the build's events: kept, since creating them
-// and copying to pageable memory took 50 us per build.
+// counts) in pinned memory, and the build's events: kept by the context, since
+// creating them and copying to pageable memory took 50 us per build.  (Kept per
+// scene, freeing the pinned words cost each scene's destruction 150-280 us, more
+// than a small scene's build.)
 struct BvhHost {
     uint32_t* p = nullptr;  // 257 words
     EventPair ev;           // the build's timing
@@ -96,7 +98,6 @@ struct BvhHost {
 
 // Scratch of the LBVH build.
 struct BvhScratch {
-    BvhHost host;
     DevBuf box_lo, box_hi;      // float4 per prim (padded boxes)
     DevBuf bounds;              // 12 ordered-u32: scene lo/hi, centroid lo/hi; deepest wide level; wide nodes
     DevBuf bpart;               // 12 ordered-u32 per block of the bounds reduction
@@ -119,7 +120,7 @@ struct BvhScratch {
 // tree collapsed from it into `wide` (8 float4 per node) on `stream`.
 // morton/order receive the sorted codes and primitive order.
 Status lbvh_build(const DevScene& sc, uint32_t n_prims, DevBuf& nodes, DevBuf& wide, DevBuf& morton, DevBuf& order,
-                  BvhScratch& scr, hipStream_t stream, aurora_bvh_stats* stats);
+                  BvhScratch& scr, BvhHost& host, hipStream_t stream, aurora_bvh_stats* stats);
 
 // Scenes of at most kFlatMaxPrims primitives also keep their leaf records in
 // Morton order (32 bytes each) for the flat traversal; flat_build fills them

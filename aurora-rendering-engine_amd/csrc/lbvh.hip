@@ -824,7 +824,7 @@ Status flat_build(uint32_t n, const DevBuf& nodes, const BvhScratch& s, DevBuf& 
 }
 
 Status lbvh_build(const DevScene& sc_in, uint32_t n, DevBuf& nodes, DevBuf& wide, DevBuf& morton, DevBuf& order,
-                  BvhScratch& s, hipStream_t st, aurora_bvh_stats* stats) {
+                  BvhScratch& s, BvhHost& host, hipStream_t st, aurora_bvh_stats* stats) {
     DevScene sc = sc_in;
     aurora_bvh_stats local{};
     local.n_prims = n;
@@ -861,8 +861,8 @@ Status lbvh_build(const DevScene& sc_in, uint32_t n, DevBuf& nodes, DevBuf& wide
     // (every internal node)
     AUR_TRY(wide.alloc(ni * 128));
 
-    AUR_TRY(s.host.create());
-    hipEvent_t e0 = s.host.ev.e[0], e1 = s.host.ev.e[1];
+    AUR_TRY(host.create());
+    hipEvent_t e0 = host.ev.e[0], e1 = host.ev.e[1];
     AUR_HIP(hipEventRecord(e0, st));
     k_prim_bounds<<<nbound, kBlock, 0, st>>>(sc, n, s.box_lo.as<float4>(), s.box_hi.as<float4>(),
                                              s.bpart.as<uint32_t>());
@@ -890,15 +890,15 @@ Status lbvh_build(const DevScene& sc_in, uint32_t n, DevBuf& nodes, DevBuf& wide
                                  s.lvl_node.as<uint32_t>(), s.hist.as<uint32_t>(), nint, 1, st));
         k_level_starts<<<1, 256, 0, st>>>(s.hist.as<uint32_t>(), blocks_for(nint, kTile), nint,
                                           s.lvl_start.as<uint32_t>());
-        uint32_t* starts = s.host.p;
+        uint32_t* starts = host.p;
         AUR_HIP(hipMemcpyAsync(starts, s.lvl_start.p, 257 * 4, hipMemcpyDeviceToHost, st));
-        AUR_HIP(hipEventRecord(s.host.starts, st));
+        AUR_HIP(hipEventRecord(host.starts, st));
         // the leaf records need no depths: they are written while the host reads these
         k_leaves<<<blocks_for(n, kBlock), kBlock, 0, st>>>(n, s.vals[0].as<uint32_t>(), s.box_lo.as<float4>(),
                                                            s.box_hi.as<float4>(), s.leaf_pos.as<uint32_t>(),
                                                            s.leaf_parent.as<uint32_t>(), s.int_pos.as<uint32_t>(),
                                                            nodes.as<float4>());
-        AUR_HIP(hipEventSynchronize(s.host.starts));
+        AUR_HIP(hipEventSynchronize(host.starts));
         if (starts[255] != nint) return Status{AURORA_ERR_RUNTIME, "LBVH build: node depths did not resolve"};
         uint32_t maxd = 0;
         for (uint32_t d = 0; d < 255; ++d)
@@ -975,7 +975,7 @@ Status lbvh_build(const DevScene& sc_in, uint32_t n, DevBuf& nodes, DevBuf& wide
     std::swap(morton, s.keys[0]);
     std::swap(order, s.vals[0]);
 
-    uint32_t* b = s.host.p;
+    uint32_t* b = host.p;
     AUR_HIP(hipMemcpyAsync(b, s.bounds.p, 14 * 4, hipMemcpyDeviceToHost, st));
     AUR_HIP(hipStreamSynchronize(st));
     if (n > 1) {

@@ -28,3 +28,36 @@ def test_build_equals_oracle_at_launch_edges(ctx, n):
         assert np.array_equal(g, w)
     assert np.array_equal(scene.nodes(), o.nodes())
     assert np.array_equal(scene.wide(), o.wide())
+
+
+def test_scenes_of_a_context_build_and_close_in_turn(ctx):
+    """The builds of a context share its pinned words: scenes of different sizes
+    built in turn each read their own counts, and a closed scene gives back only
+    device memory, in less time than half its build took (a pinned free per scene
+    took longer than the build)."""
+    import time
+    arrs = [scenes.batch_scene(n, n, n)[0] for n in (2, 5, 100, 3000)]
+    want = []
+    for arr in arrs:
+        o = orc.OracleScene(arr)
+        want.append(o.build_bvh())
+    up = [ctx.upload(a) for a in arrs]
+    for order in ((0, 1, 2, 3), (3, 1, 0, 2)):
+        for k in order:
+            got = up[k].build_bvh()
+            for key in ("n_prims", "n_nodes", "n_wide", "depth", "wide_depth", "scene_lo", "scene_hi"):
+                assert got[key] == want[k][key], (k, key)
+    for s in up:
+        s.close()
+    build, many = [], [ctx.upload(arrs[2]) for _ in range(32)]
+    for s in many:
+        s.build_bvh()
+        t0 = time.perf_counter()
+        s.build_bvh()
+        build.append(time.perf_counter() - t0)
+    t0 = time.perf_counter()
+    for s in many:
+        s.close()
+    close = (time.perf_counter() - t0) / len(many)
+    print("100 primitives: build", np.median(build), "close", close, flush=True)
+    assert close < 0.5 * np.median(build)
