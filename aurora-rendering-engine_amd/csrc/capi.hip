@@ -62,6 +62,7 @@ struct aurora_ctx {
     BvhHost bvh_host;                // the LBVH builds' pinned words and events
     uint32_t host_recs_cap = 0;
     unsigned char* scratch = nullptr;  // this device's copy of the allocation-free scratch array
+    DevBuf na_pool;                    // work counters of the allocation-free queries
     PatchWork patch;                   // patch-projection renderer tables
 };
 
@@ -84,29 +85,32 @@ struct aurora_scene {
 // aurora_trace_closest_device_noalloc keeps every buffer beyond the caller's
 // rays and hits in `scratch`, a static device array of which each GPU holds
 // its own copy until the process ends: the packed rays and hits of up to
-// kNoAllocMaxRays rays, the work-pool counters, the one-entry scene table and
-// the traversal stack spill of a grid of at most kNoAllocGrid blocks.  Host
+// kNoAllocMaxRays rays, the one-entry scene table and the traversal stack spill
+// of a grid of at most kNoAllocGrid blocks (the work counters are the context's,
+// from its creation on).  Host
 // code never passes the array's name to a kernel (on the host it is only a
 // stand-in): its device address is taken once per device with
 // hipGetSymbolAddress (scratch_address, called by aurora_create) and kept
 // in the context.
 constexpr uint32_t kNoAllocMaxRays = AURORA_NOALLOC_MAX_RAYS;
-constexpr int kNoAllocGrid = 511;  // about two 256-thread blocks per CU
+// Two 256-thread blocks per CU.  The largest call then gives every lane the same
+// number of rays: with one block less, which leaves a few rays for a third turn,
+// 262,144 counted rays took 1147 us instead of 988 on 190 k overlapping
+// primitives, and 6020 instead of 4885 on 1.2 M.
+constexpr int kNoAllocGrid = 512;
+static_assert(kNoAllocMaxRays % (kNoAllocGrid * kExtendBlock) == 0, "the largest call fills every turn of the grid");
 constexpr size_t kNaRayBytes = (size_t)kNoAllocMaxRays * 16;  // float4 per ray, origins then directions
 constexpr size_t kNaHitBytes = (size_t)kNoAllocMaxRays * 8;   // float2 (t, prim) per ray
-constexpr size_t kNaPoolBytes = (size_t)kPools * kPoolStride * 4;
 constexpr size_t kNaRecBytes = 1024;
-constexpr size_t kNaSpillBytes = (size_t)kNoAllocGrid * kExtendBlock * 80 * 4;
+constexpr size_t kNaSpillBytes = (size_t)kNoAllocGrid * kExtendBlock * kExtendSpillLevels * 4;
 constexpr size_t kNaOffDir = kNaRayBytes;
 constexpr size_t kNaOffHit = 2 * kNaRayBytes;
-constexpr size_t kNaOffPool = kNaOffHit + kNaHitBytes;
-constexpr size_t kNaOffRec = kNaOffPool + kNaPoolBytes;
+constexpr size_t kNaOffRec = kNaOffHit + kNaHitBytes;
 constexpr size_t kNaOffSpill = kNaOffRec + kNaRecBytes;
 constexpr size_t kNoAllocScratchBytes = AURORA_NOALLOC_SCRATCH_BYTES;
 static_assert(kNaOffSpill + kNaSpillBytes <= kNoAllocScratchBytes, "scratch size stated in aurora.h");
 static_assert(sizeof(SceneRec) <= kNaRecBytes, "scene record fits its slot");
-static_assert(kNaOffDir % 256 == 0 && kNaOffHit % 256 == 0 && kNaOffPool % 256 == 0 && kNaOffRec % 256 == 0 &&
-                  kNaOffSpill % 256 == 0,
+static_assert(kNaOffDir % 256 == 0 && kNaOffHit % 256 == 0 && kNaOffRec % 256 == 0 && kNaOffSpill % 256 == 0,
               "scratch regions 256-byte aligned");
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
@@ -1011,6 +1015,7 @@ int aurora_create(int device, aurora_ctx** out) {
         return fail(nullptr, s);
     }
     if (!s.bad()) s = scratch_address(device, &c->scratch);
+    if (!s.bad()) s = c->na_pool.alloc(kPools * kPoolStride * 4);
     if (s.bad()) {
         for (int k = 0; k < 2; ++k)
             if (c->recs_ev[k]) (void)hipEventDestroy(c->recs_ev[k]);
@@ -1030,7 +1035,7 @@ void aurora_destroy(aurora_ctx* c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     Workspace& w = c->ws;
     DevBuf* bufs[] = {&w.q_o[0], &w.q_o[1], &w.q_d[0], &w.q_d[1], &w.q_b[0], &w.q_b[1], &w.hit, &w.L,
-                      &w.aov_a, &w.aov_n, &w.counters, &w.spill, &w.recs};
+                      &w.aov_a, &w.aov_n, &w.counters, &w.spill, &w.recs, &c->na_pool};
     for (DevBuf* b : bufs) b->release();
     c->patch.release();
     if (w.host_counts) (void)hipHostFree(w.host_counts);
@@ -1286,7 +1291,7 @@ int aurora_trace_closest_device_noalloc(aurora_scene* s, const float* o, const f
     float4* ro = reinterpret_cast<float4*>(base);
     float4* rd = reinterpret_cast<float4*>(base + kNaOffDir);
     float2* hit = reinterpret_cast<float2*>(base + kNaOffHit);
-    uint32_t* pool = reinterpret_cast<uint32_t*>(base + kNaOffPool);
+    uint32_t* pool = c->na_pool.as<uint32_t>();
     SceneRec* rec = reinterpret_cast<SceneRec*>(base + kNaOffRec);
     uint32_t* spill = reinterpret_cast<uint32_t*>(base + kNaOffSpill);
     const uint32_t blocks = (n + 255) / 256;

@@ -323,8 +323,8 @@ int aurora_trace_closest_device_stats(aurora_scene* scene,
  * synchronisation; every buffer beyond the caller's rays, hits and counts
  * lives in a static device array of AURORA_NOALLOC_SCRATCH_BYTES (50 MiB)
  * that each GPU the library runs on holds until the process ends (packed
- * rays and hits, work counters, the scene table, the traversal stack
- * spill).  At most AURORA_NOALLOC_MAX_RAYS rays per call (more:
+ * rays and hits, the scene table, the traversal stack spill), or was allocated
+ * with the context (work counters).  At most AURORA_NOALLOC_MAX_RAYS rays per call (more:
  * AURORA_ERR_INVALID); rays are traced in the given order (the
  * aurora_set_ray_sort mode does not apply).  Asynchronous on the context
  * stream.  Every call on one GPU shares that GPU's array: calls that
