@@ -37,6 +37,7 @@ constexpr uint32_t kSortMinNodes = 1u << 21;
 // overlapping 10.0 -> 7.4)
 constexpr uint32_t kGroupMinPrims = 16384;
 constexpr uint32_t kFlatDefaultPrims = 64;
+constexpr int kGroupBlocksPerCu = 8;  // resident blocks of the group walk
 
 struct aurora_ctx {
     int device = 0;
@@ -98,6 +99,8 @@ constexpr uint32_t kNoAllocMaxRays = AURORA_NOALLOC_MAX_RAYS;
 // 262,144 counted rays took 1147 us instead of 988 on 190 k overlapping
 // primitives, and 6020 instead of 4885 on 1.2 M.
 constexpr int kNoAllocGrid = 512;
+// four blocks per CU of the group walk, whose spill is less than half per thread
+constexpr int kNoAllocGroupGrid = 1024;
 static_assert(kNoAllocMaxRays % (kNoAllocGrid * kExtendBlock) == 0, "the largest call fills every turn of the grid");
 constexpr size_t kNaRayBytes = (size_t)kNoAllocMaxRays * 16;  // float4 per ray, origins then directions
 constexpr size_t kNaHitBytes = (size_t)kNoAllocMaxRays * 8;   // float2 (t, prim) per ray
@@ -109,6 +112,8 @@ constexpr size_t kNaOffRec = kNaOffHit + kNaHitBytes;
 constexpr size_t kNaOffSpill = kNaOffRec + kNaRecBytes;
 constexpr size_t kNoAllocScratchBytes = AURORA_NOALLOC_SCRATCH_BYTES;
 static_assert(kNaOffSpill + kNaSpillBytes <= kNoAllocScratchBytes, "scratch size stated in aurora.h");
+static_assert((size_t)kNoAllocGroupGrid * kGroupBlockRays * kGroupSpillBytes <= kNaSpillBytes,
+              "the group walk's spill fits");
 static_assert(sizeof(SceneRec) <= kNaRecBytes, "scene record fits its slot");
 static_assert(kNaOffDir % 256 == 0 && kNaOffHit % 256 == 0 && kNaOffRec % 256 == 0 && kNaOffSpill % 256 == 0,
               "scratch regions 256-byte aligned");
@@ -382,8 +387,10 @@ Status trace_device(aurora_scene* s, const float* o, const float* d, uint32_t n,
     if (n == 0) return Status::ok();
     const uint32_t blocks = (n + 255) / 256;
     if (!brute && !counts && !count_fetches) {
-        // no counters: the group walk on the caller's rays and hits
-        const int grid = grid_for_group(c, n);
+        // no counters: walked on the caller's rays and hits
+        const int group_grid = grid_for_group(c, n), lane_grid = grid_for_extend(c, n);
+        const QueryWalk walk = query_walk(
+            n, s->n_prims, (uint32_t)(std::min(c->ext_grid, c->cus * kGroupBlocksPerCu) * kGroupBlockRays));
         if (hits_over_rays(o, d, prim, t, n)) {
             AUR_TRY(s->tr_o.alloc((size_t)n * 16));
             AUR_TRY(s->tr_d.alloc((size_t)n * 16));
@@ -400,9 +407,10 @@ Status trace_device(aurora_scene* s, const float* o, const float* d, uint32_t n,
         q.tmax = tmax;
         q.prim = prim;
         q.t = t;
-        AUR_TRY(ensure_spill(s->tr_spill, grid));
+        q.box = s->view.nodes;
+        AUR_TRY(s->tr_spill.alloc(std::max(query_spill_bytes(QueryWalk::Group, group_grid),
+                                           walk == QueryWalk::Group ? 0 : query_spill_bytes(QueryWalk::Lanes, lane_grid))));
         q.spill = s->tr_spill.as<uint32_t>();
-        q.spill_stride = (uint32_t)(grid * extend_block());
         AUR_TRY(s->tr_pool.alloc(kPools * kPoolStride * 4));
         q.pool = s->tr_pool.as<uint32_t>();
         const bool sort = s->stats.n_nodes > 0 &&
@@ -428,7 +436,7 @@ Status trace_device(aurora_scene* s, const float* o, const float* d, uint32_t n,
                                      s->tr_key[1].as<uint32_t>(), s->tr_val[1].as<uint32_t>(),
                                      s->tr_hist.as<uint32_t>(), n, 4, c->stream));
         }
-        AUR_TRY(launch_query(q, grid, c->stream));
+        AUR_TRY(launch_query(q, walk, group_grid, lane_grid, c->stream));
         if (ts) {
             AUR_HIP(hipEventRecord(ev.e[1], c->stream));
             AUR_HIP(hipEventSynchronize(ev.e[1]));
@@ -1311,9 +1319,11 @@ int aurora_trace_closest_device_noalloc(aurora_scene* s, const float* o, const f
         q.pool = pool;
         q.prim = prim;
         q.t = t;
+        q.box = s->view.nodes;
         q.spill = spill;
-        q.spill_stride = (uint32_t)kNoAllocGrid * kExtendBlock;
-        CK(c, launch_query(q, std::min(grid_for_group(c, n), kNoAllocGrid), c->stream));
+        const QueryWalk walk = query_walk(n, s->n_prims, kNoAllocGroupGrid * kGroupBlockRays);
+        const int group_grid = (int)std::min<uint32_t>((n + kGroupBlockRays - 1) / kGroupBlockRays, kNoAllocGroupGrid);
+        CK(c, launch_query(q, walk, group_grid, std::min(grid_for_extend(c, n), kNoAllocGrid), c->stream));
         return AURORA_OK;
     }
     k_pack3<<<blocks, 256, 0, c->stream>>>(o, ro, n);

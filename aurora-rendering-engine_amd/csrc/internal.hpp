@@ -170,6 +170,12 @@ struct GroupScene {
     float tmin;
 };
 constexpr int kGroupBlockRays = 64;  // rays that a block of a group walk holds
+constexpr int kGroupSpillBytes = 608;  // stack spill of a ray of a group walk
+// How a query walks: four lanes per ray, one lane per ray, or whichever suits the
+// rays, decided on the device (query_walk, trace.hip).
+enum class QueryWalk { Group, Lanes, Pick };
+// groups: the rays that the group walk's grid holds at once
+QueryWalk query_walk(uint32_t n, uint32_t n_prims, uint32_t groups);
 // Closest hits of n rays given as packed floats, into prim and t.
 struct QueryArgs {
     const float *org, *dir;   // 3 per ray
@@ -177,13 +183,18 @@ struct QueryArgs {
     GroupScene sc;
     float tmax;
     const uint32_t* order;    // optional: claim order of the rays (slot -> ray index)
-    uint32_t* pool;           // kPools work counters kPoolStride u32 apart (set to 0 by launch_query when used)
+    const float4* box;        // the scene's box (lo, hi), for Pick
+    uint32_t* pool;           // kPools work counters kPoolStride u32 apart (set by launch_query)
+    uint32_t pick;            // set by launch_query
     int32_t* prim;
     float* t;
-    uint32_t* spill;          // as in ExtendArgs
-    uint32_t spill_stride;
+    uint32_t* spill;          // query_spill_bytes of both grids
+    uint32_t spill_stride;    // set by launch_query: threads of the grid
 };
-Status launch_query(const QueryArgs& a, int grid, hipStream_t stream);
+// the stack spill of a walk on a grid of so many blocks
+size_t query_spill_bytes(QueryWalk walk, int blocks);
+// group_grid, lane_grid: blocks of the two walks (the one not taken is not read)
+Status launch_query(const QueryArgs& a, QueryWalk walk, int group_grid, int lane_grid, hipStream_t stream);
 Status launch_brute(const DevScene& sc, const float4* o, const float4* d, uint32_t n, float tmin, float tmax,
                     float2* hit, hipStream_t stream);
 // Sort keys of n rays for traversal order: 27-bit Morton code of the origin

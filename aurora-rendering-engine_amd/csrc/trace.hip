@@ -4,8 +4,9 @@
 // Two persistent kernels, both over grids sized to the resident capacity of
 // the chip, whose waves claim rays from WaveClaims' counters:
 //   k_query / k_extend_group  the group walk (traverse.hpp): four lanes per ray
-//     on the four-wide tree.  Every uncounted ray query, and the bounces of
-//     renders of larger scenes.
+//     on the four-wide tree.  Uncounted ray queries, but those of many rays on
+//     small scenes (k_query_lanes, one lane per ray; query_walk says which), and
+//     the bounces of renders of larger scenes.
 //   k_extend  one lane per ray: the binary tree (render bounces), the four-wide
 //     tree for small scenes' bounces, and every run that counts fetches (their
 //     counts are those of this visit order).  When enough lanes of a wave64
@@ -17,14 +18,15 @@
 //     hit 64 consecutive banks) and spills deeper levels to a per-thread global
 //     array.
 //
-// What the group walk gave (queries, one lane per ray before -> after): 2^20
-// sorted rays on 1.2 M overlapping primitives 11.9 -> 6.2 ms; 10^6 rays on 190 k
-// primitives 0.70 -> 0.51 ms, on 488 spheres 0.24 -> 0.15; 10^5 rays on 50 k
-// primitives 210 -> 115 us; 1000 rays 57 -> 13 us (of which the packing kernels
-// and the upload of a scene record, with its synchronisation, were 40).  It is
-// bound by VALU issue (one wave instruction per SIMD and 4 cycles: 4.26e9 in
-// 6.6 ms, with 52 of 64 lanes active; 27 of 64 before, when the L1 address path
-// was busy 75% of the time).
+// What the group walk gave (queries of random rays in a row, one lane per ray
+// before -> after): 2^20 sorted rays on 1.2 M overlapping primitives 12.0 -> 6.4
+// ms; 2^20 rays on 190 k scattered primitives 0.80 -> 0.54 ms; 100,001 rays on a
+// serving scene of 50 k 226 -> 67 us; 1000 rays on 485 spheres 73 -> 5 us (13 us for
+// one call alone), of which the packing kernels and the upload of a scene record,
+// with its synchronisation, were 40.  The first of these issues 4.26e9 VALU
+// instructions at 645 G/s (one kind alone reaches 614 G/s, pairs 1229) with 52 of
+// 64 lanes active; 27 of 64 before, when the L1 address path was busy 75% of the
+// time.
 //
 // Reference counterpart: the per-ray linear scan over all triangles,
 // experiments/rt.cpp:209-218, with are::Triangle::intersect_ray
@@ -40,6 +42,7 @@ constexpr int kBlock = 256;
 constexpr int kLds = 16;
 constexpr int kMaxStack = 96;  // three pushes per level of a tree of depth <= 64
 constexpr int kRefill = 8;
+constexpr uint32_t kPickWord = 1;  // of the work counters (which are kPoolStride apart): the walk that k_query_pick took
 constexpr uint32_t kNone = 0xffffffffu;
 constexpr uint32_t kNoPrim = 0x7fffffffu;
 
@@ -376,7 +379,83 @@ struct QueryIO {
     }
 };
 __global__ __launch_bounds__(kBlock) void k_query(QueryArgs a) {
+    if (a.pick && a.pool[kPickWord] != 0u) return;
     group_trace(QueryIO{a}, a.n, a.pool, a.tmax, a.spill, a.spill_stride);
+}
+
+// The same with one lane per ray.  Where the rays of a wave go the same way its
+// 64 lanes walk together, and the group walk's four lanes per ray only give the
+// wave a quarter of the rays (query_walk has the figures).
+__global__ __launch_bounds__(kBlock) void k_query_lanes(QueryArgs a) {
+    if (a.pick && a.pool[kPickWord] == 0u) return;
+    __shared__ uint32_t stk[kTravLds * kBlock];
+    const QueryIO io{a};
+    uint32_t* spill = a.spill + (size_t)blockIdx.x * kBlock + threadIdx.x;
+    DevScene sc{};
+    sc.wide = a.sc.wide;
+    sc.spheres = a.sc.spheres;
+    sc.quads = a.sc.quads;
+    sc.n_wide = a.sc.n_wide;
+    sc.n_spheres = a.sc.n_spheres;
+    sc.n_quads = a.sc.n_prims - a.sc.n_spheres;
+    uint32_t ri = kNone;
+    bool done = false;
+    v3 o = V(0, 0, 0), d = V(0, 0, 0);
+    WideWalk w{};
+    WaveClaims claims;
+    claims.init(a.pool, a.n, 64u, 0u);
+    for (;;) {
+        const bool idle = (ri == kNone) && !done;
+        const uint64_t im = __ballot(idle);
+        const uint64_t am = __ballot(ri != kNone);
+        if (im != 0 && (am == 0 || __popcll(im) >= kRefill)) {
+            claims.refill();
+            const uint32_t avail = claims.next < claims.end ? claims.end - claims.next : 0u;
+            const uint32_t rank = lanes_below(im);
+            if (idle) {
+                if (avail == 0) {
+                    done = true;
+                } else if (rank < avail) {
+                    uint32_t sid = 0u;
+                    ri = io.ray(claims.next + rank, o, d, sid);
+                    wide_walk_start(w, d, a.tmax);
+                }
+            }
+            claims.next += min(avail, (uint32_t)__popcll(im));
+        }
+        if (__ballot((ri != kNone) || !done) == 0) break;
+        if (ri == kNone) continue;
+        if (wide_walk_step(w, sc, o, d, a.sc.tmin, a.tmax, stk + threadIdx.x, kBlock, spill, a.spill_stride)) {
+            float t;
+            int prim;
+            wide_walk_result(w, a.tmax, t, prim);
+            io.hit(ri, t, prim);
+            ri = kNone;
+        }
+    }
+}
+
+// Clears the work counters and decides which of the two walks runs: 1024 pairs of
+// rays that a wave would hold together, 31 places apart in claim order; lanes when
+// three quarters of them start within a sixteenth of the scene's extent and go
+// within 8 degrees (a pinhole image's neighbours do, also past the ends of its
+// rows; random, bounced or shadow rays of an area light do not).
+__global__ __launch_bounds__(1024) void k_query_pick(QueryArgs a) {
+    const uint32_t i = threadIdx.x;
+    if (i < kPools) a.pool[kPoolStride * i] = 0u;
+    const QueryIO io{a};
+    const uint32_t p = (uint32_t)(((uint64_t)a.n * i) / 1024u);
+    v3 o0, d0, o1, d1;
+    uint32_t sid = 0u;
+    (void)io.ray(p, o0, d0, sid);
+    (void)io.ray(min(a.n - 1u, p + 31u), o1, d1, sid);
+    const float4 lo = a.box[0], hi = a.box[1];
+    const float reach = fmaxf(fmaxf(hi.x - lo.x, hi.y - lo.y), hi.z - lo.z) * 0.0625f;
+    const v3 s = o1 - o0;
+    const float c = dot(d0, d1);
+    const bool same = dot(s, s) <= reach * reach && c > 0.0f && (c * c >= 0.98f * dot(d0, d0) * dot(d1, d1));
+    const int n_same = __syncthreads_count(same);
+    if (i == 0) a.pool[kPickWord] = n_same >= 768 ? 1u : 0u;
 }
 
 // the live queue of a wavefront bounce
@@ -503,15 +582,51 @@ Status launch_extend(const ExtendArgs& a, int grid, hipStream_t s) {
     return Status::ok();
 }
 
-Status launch_query(const QueryArgs& args, int grid, hipStream_t s) {
+// Which walk a query takes (us; camera: the rays of a 512x512 pinhole image,
+// random: 262,144 and 2^20 rays of random origin and direction).
+// - As many rays as the group walk's grid holds, or fewer: group.  The call is
+//   as long as its longest ray, and four lanes shorten it: 10^5 camera rays on 500,
+//   8 k and 50 k primitives 26, 52, 88 against 73, 118, 168 by lanes (packing them),
+//   random ones 33, 74, 123 against 98, 157, 241.
+// - Fewer than 1,024 primitives: lanes.  500 primitives: camera 120 by groups, 62 by
+//   lanes; random 107 and 239, 88 and 211.
+// - 32,768 or more: group.  50 k primitives: camera 174 and, by lanes, 209; random 211
+//   and 443, 295 and 592.
+// - Between these, lanes where the rays of a wave go the same way and groups where
+//   they do not.  2,000 primitives: camera 155 by groups, 82 by lanes; 2^21 random
+//   rays 449 and 486.  8,000: camera 175 and 125; random 161 and 335, 201 and 430.
+//   The look at the rays and the idle walk's launch cost 3 to 8 us.
+constexpr uint32_t kLaneAlwaysPrims = 1024, kLaneMaxPrims = 32768;
+QueryWalk query_walk(uint32_t n, uint32_t n_prims, uint32_t groups) {
+    if (n <= groups || n_prims >= kLaneMaxPrims) return QueryWalk::Group;
+    return n_prims < kLaneAlwaysPrims ? QueryWalk::Lanes : QueryWalk::Pick;
+}
+
+size_t query_spill_bytes(QueryWalk walk, int blocks) {
+    return walk == QueryWalk::Lanes ? (size_t)blocks * kBlock * (kTravMaxStack - kTravLds) * 4
+                                    : (size_t)blocks * kGroupBlockRays * kGroupSpillBytes;
+}
+static_assert(kGroupSpillBytes == (kGroupMaxStack - kGroupStack) * 8 &&
+                  kGroupBlockRays * kGroupSpillBytes <= kBlock * kExtendSpillLevels * 4,
+              "group spill: no more than k_extend_group's share of ExtendArgs::spill");
+
+Status launch_query(const QueryArgs& args, QueryWalk walk, int group_grid, int lane_grid, hipStream_t s) {
     QueryArgs a = args;
-    if ((size_t)grid * kBlock > a.spill_stride) return Status{AURORA_ERR_RUNTIME, "query grid exceeds spill stride"};
-    if ((uint64_t)grid * kGroupBlockRays >= a.n) {
+    a.pick = walk == QueryWalk::Pick ? 1u : 0u;
+    if (walk == QueryWalk::Group && (uint64_t)group_grid * kGroupBlockRays >= a.n)
         a.pool = nullptr;  // one ray per place: nothing to claim
-    } else {
+    else if (a.pick)
+        k_query_pick<<<1, 1024, 0, s>>>(a);
+    else
         k_clear_pool<<<1, 64, 0, s>>>(a.pool);
+    if (walk != QueryWalk::Group) {
+        a.spill_stride = (uint32_t)(lane_grid * kBlock);
+        k_query_lanes<<<lane_grid, kBlock, 0, s>>>(a);
     }
-    k_query<<<grid, kBlock, 0, s>>>(a);
+    if (walk != QueryWalk::Lanes) {
+        a.spill_stride = (uint32_t)(group_grid * kBlock);
+        k_query<<<group_grid, kBlock, 0, s>>>(a);
+    }
     AUR_HIP(hipGetLastError());
     return Status::ok();
 }
