@@ -5,8 +5,8 @@ shape, and the fastest is kept and cached under a signature of the
 workload (pixels, samples, primitives).  The shape covers the persistent
 traversal and shading grids (blocks per compute unit), the live-path count
 at which the fused tail takes over, whether passes are captured in a
-hipGraph, which tree (binary, four-wide, or the flat leaf array of a small
-scene) the render kernels walk, and the queue sizes: the most paths per
+hipGraph, which tree (the library's choice, four-wide, or the flat leaf array
+of a small scene) the render kernels walk, and the queue sizes: the most paths per
 pass and the paths a wave claims per work-pool atomic (candidates add them
 as "pass_paths" / "claim_paths"; 0 is the library's choice).
 Shapes change speed only, never results (tests check the images bit for
@@ -29,8 +29,8 @@ CANDIDATES = {
 
 
 def tree_of(shape):
-    """The render tree of a shape: its "tree" (0 binary, 1 four-wide, 2 flat),
-    or its "wide" flag."""
+    """The render tree of a shape: its "tree" (Context.set_render_tree: 0 the
+    library's choice, 1 four-wide, 2 flat, 3 binary), or its "wide" flag."""
     return int(shape["tree"]) if "tree" in shape else (1 if shape.get("wide", False) else 0)
 
 

@@ -181,11 +181,11 @@ class Context:
         self.check(self.lib.aurora_set_launch(self.h, extend_blocks_per_cu, shade_blocks_per_cu, tail_paths))
 
     def set_render_tree(self, tree=0):
-        """Tree the render kernels walk: 0 (or False) the binary LBVH
-        (default; flat for one small scene of large overlapping primitives), 1
-        (or True) the four-wide tree, 2 the flat leaf array of a
-        small scene (single-scene renders; four-wide elsewhere).  Speed only;
-        the images are the same."""
+        """Tree the render kernels walk: 0 (or False) the library's choice
+        (default: the binary LBVH, flat for one small scene of large overlapping
+        primitives), 1 (or True) the four-wide tree, 2 the flat leaf array of a
+        small scene (single-scene renders; four-wide elsewhere), 3 the binary
+        LBVH in every case.  Speed only; the images are the same."""
         self.check(self.lib.aurora_set_render_tree(self.h, int(tree)))
 
     def selftest_rcp(self, lo, hi):

@@ -36,7 +36,26 @@ constexpr uint32_t kSortMinNodes = 1u << 21;
 // 1000 primitives 2.2 -> 2.5, 50 k 7.1 -> 6.4, 190 k 10.4 -> 9.2, 800 k
 // overlapping 10.0 -> 7.4)
 constexpr uint32_t kGroupMinPrims = 16384;
-constexpr uint32_t kFlatDefaultPrims = 64;
+// The default tree's flat walk: one scene of few leaves whose boxes a ray enters
+// at least one of on average (overlap: flat_build's), where a tree has little to
+// cull.  Times of the flat walk over the binary one, scattered scenes scaled to the
+// overlap, depth 50 (depth 8 and 1 sample in small passes):
+// - passes of up to 32,768 paths are as long as one wave's paths: 0.58 to 0.98 at
+//   every size and overlap >= 1 (160x120: the Cornell box, 18 leaves, overlap 2.4,
+//   139 -> 94 us); at 65,536 up to 1.05.
+// - larger passes, 10 to 32 leaves: 0.51 to 1.04 (Cornell 1024x640, 8 samples, 2.32
+//   -> 1.48 ms); 40 leaves 0.84 to 1.01 from overlap 1.25 on, 1.09 at 1.0; 48 to 64
+//   leaves up to 1.21 at 1.25 and 1.15 at 1.7; 2 to 8 leaves up to 1.22.
+// - overlap below 1: 1.03 to 1.3; more than 64 leaves: 1.58 for 200 at overlap 3.
+constexpr bool flat_default(uint32_t prims, float overlap, uint64_t pass_paths) {
+    if (prims > 64 || !(overlap >= 1.0f)) return false;
+    return pass_paths <= 32768 || (prims >= 10 && prims <= 40 && 32.0f * overlap >= (float)prims);
+}
+static_assert(flat_default(18, 2.4f, 33554432) && flat_default(10, 1.0f, 65536) && flat_default(40, 1.25f, 65536), "");
+static_assert(!flat_default(64, 1.04f, 5242880) && !flat_default(64, 1.7f, 655360) && !flat_default(40, 1.01f, 655360), "");
+static_assert(!flat_default(4, 1.2f, 655360) && !flat_default(9, 2.0f, 32769), "");
+static_assert(flat_default(4, 1.2f, 32768) && flat_default(64, 1.0f, 19200), "");
+static_assert(!flat_default(65, 3.0f, 19200) && !flat_default(18, 0.99f, 19200), "");
 constexpr int kGroupBlocksPerCu = 8;  // resident blocks of the group walk
 
 struct aurora_ctx {
@@ -49,7 +68,8 @@ struct aurora_ctx {
     uint32_t tail_paths = 0xffffffffu;  // fused-tail switch: live paths at or below (default: always)
     uint32_t graph_tail_depth = 8;   // captured passes switch to the fused tail here
     int ray_sort = 1;                // ray queries: 0 never sort, 1 large scenes, 2 always
-    uint32_t render_tree = 0;        // render bounces: 0 binary LBVH, 1 four-wide tree, 2 flat (small scenes)
+    uint32_t render_tree = 0;        // render bounces: binary LBVH, 1 four-wide tree, 2 flat (small scenes)
+    bool flat_auto = true;           // render_tree 0: flat where flat_default says so
     uint64_t pass_paths = 0;         // automatic passes: at most this many paths (0: kPassPaths)
     uint32_t claim_paths = 0;        // fused-tail paths per pool claim (0: by pass size)
     Workspace ws;                    // path queues shared by the context's renders
@@ -654,16 +674,10 @@ Status render_jobs(aurora_ctx* c, std::vector<Job>& jobs, aurora_render_stats* s
     // the fused tail is persistent: its grid is the resident capacity
     // the passes walk the flat leaf array under the condition render_jobs
     // sets pa.flat by (one scene, small enough to have the array)
-    // (the default tree too where a tree has little to cull: few leaves, whose
-    // boxes a ray enters at least one of on average.  160x120, 1 sample, depth
-    // 8 / 1024x640, 8 samples, depth 50, binary -> flat: the Cornell box, 18
-    // leaves, overlap 2, 215 -> 165 us / 2.41 -> 1.60 ms; scattered scenes of
-    // overlap below 1: 10 leaves 151 -> 143 us / 1.20 -> 1.24 ms, 30 leaves 168 ->
-    // 169 / 1.19 -> 1.25, 120 leaves 202 -> 248 / 1.58 -> 2.07)
     const bool flat =
         jobs.size() == 1 && jobs[0].scene->view.n_flat > 0 &&
-        (c->render_tree == 2 || (c->render_tree == 0 && jobs[0].scene->n_prims <= kFlatDefaultPrims &&
-                                 jobs[0].scene->flat_overlap >= 1.0f));
+        (c->render_tree == 2 || (c->render_tree == 0 && c->flat_auto &&
+                                 flat_default(jobs[0].scene->n_prims, jobs[0].scene->flat_overlap, cap)));
     // four-wide wavefront bounces: the group walk where most paths are in
     // scenes of at least kGroupMinPrims primitives, one lane per ray elsewhere
     uint64_t big = 0, all = 0;
@@ -1089,9 +1103,10 @@ int aurora_set_queue(aurora_ctx* c, uint32_t pass_paths, uint32_t claim_paths) {
 
 int aurora_set_render_tree(aurora_ctx* c, int tree) {
     if (!c) return fail(nullptr, AURORA_ERR_INVALID, "ctx is NULL");
-    if (tree < 0 || tree > 2)
-        return fail(c, AURORA_ERR_INVALID, "render tree must be 0 (binary), 1 (four-wide) or 2 (flat)");
-    c->render_tree = (uint32_t)tree;
+    if (tree < 0 || tree > 3)
+        return fail(c, AURORA_ERR_INVALID, "render tree must be 0 (default), 1 (four-wide), 2 (flat) or 3 (binary)");
+    c->flat_auto = tree == 0;
+    c->render_tree = tree == 3 ? 0u : (uint32_t)tree;
     return AURORA_OK;
 }
 

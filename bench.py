@@ -726,11 +726,11 @@ def main():
         best, tune_table = autotune.tune(ctx, tune_run, f"cornell_{W}x{H}_spp{S}", cache_path=None, log=note,
                                          candidates={"extend_blocks_per_cu": [8], "shade_blocks_per_cu": [8],
                                                      "tail_paths": [1 << 20, TAIL_ALWAYS],
-                                                     "graph": [False], "tree": [0, 1, 2]})
+                                                     "graph": [False], "tree": [3, 1, 2]})
         graph = best["graph"]
         shape = {k: best[k] for k in best if k != "seconds"}
     else:
-        tree = {"binary": 0, "wide": 1, "flat": 2}[args.render_tree]
+        tree = {"binary": 3, "wide": 1, "flat": 2}[args.render_tree]
         ctx.set_render_tree(tree)
         shape = {"tail_paths": args.tail_paths, "tree": tree}
 

@@ -241,14 +241,15 @@ int aurora_set_launch(aurora_ctx* ctx, int extend_blocks_per_cu,
  * decide which lane carries which path. */
 int aurora_set_queue(aurora_ctx* ctx, uint32_t pass_paths, uint32_t claim_paths);
 
-/* Tree walked by the render kernels: 0 = the binary LBVH (default; one
- * 64-byte child pair per step; the persistent path kernel takes the flat form
- * for a single scene of at most 64 primitives whose leaf boxes' areas add up to
- * the scene box's, such as a small closed room), 1 = the four-wide tree (one
- * 128-byte node per step), 2 = flat: for single-scene renders of scenes of at most 256
- * primitives, the persistent path kernel tests every leaf in Morton order,
+/* Tree walked by the render kernels: 0 = the library's choice (default): the
+ * binary LBVH, but the flat form in the persistent path kernel for a single
+ * scene of few primitives whose leaf boxes' areas add up to the scene box's,
+ * such as a small closed room; 1 = the four-wide tree (one 128-byte node per
+ * step); 2 = flat: for single-scene renders of scenes of at most 256
+ * primitives, the persistent path kernel tests every leaf, largest box first,
  * the same sequence for every ray (no stack, no divergence); elsewhere 2
- * walks the four-wide tree.  Which is fastest depends on the scene (the
+ * walks the four-wide tree; 3 = the binary LBVH (one 64-byte child pair per
+ * step) in every case.  Which is fastest depends on the scene (the
  * autotuner tries them); the images are the same.  No reference
  * counterpart. */
 int aurora_set_render_tree(aurora_ctx* ctx, int tree);
