@@ -1,7 +1,7 @@
 """The denoiser at image sizes where its tiles end: the smallest image, widths
 past a 64-pixel segment by 8 pixels, a coarsest level of one pixel, batches,
-and a size whose full resolution takes two rows per wave with a ragged last
-segment.  Same references and bounds as test_gpu_denoiser.py."""
+a size whose full resolution takes two rows per wave with a ragged last segment,
+and one whose every level does.  Same references and bounds as test_gpu_denoiser.py."""
 import numpy as np
 import pytest
 import torch
@@ -50,3 +50,30 @@ def test_gradient_edges(ctx, B, H, W):
     assert np.linalg.norm(g - gr) / np.linalg.norm(gr) < 0.1
     # fixed summation order: the same gradients again
     assert np.array_equal(net.loss_grad(*args, spp)[1], g)
+
+
+def test_forward_pools_in_the_convolution_at_every_level(ctx):
+    """The smallest square image whose level 2 (64 channels) pools in its
+    convolution's epilogue (512 blocks of 8 rows x 64 pixels), and one 32 rows
+    shorter, where a kernel of its own pools that level: crops of both match the
+    reference, with the bounds of the other forward tests."""
+    net = dn.Denoiser(ctx, seed=1)
+    p = random_params(net.n, 13)
+    net.set_params(p)
+    spp, W = 4, 2048
+    rgb, alb, nrm, _ = inputs(1, 2048, W, seed=21, spp=spp)
+    for H in (2048, 2016):
+        a = [t[0, :H].contiguous() for t in (rgb, alb, nrm)]
+        out = net.denoise(*[t.cuda() for t in a], spp).cpu().numpy()
+        # the receptive field of a pixel reaches less than 96 pixels: the reference on a crop
+        # is the image's where the crop's edge is that far away or the image's own
+        for y0, x0 in ((0, 0), (H - 384, W - 384), (H // 16 * 8, 1024)):
+            y1, x1 = y0 + 384, x0 + 384
+            crop = [t[None, y0:y1, x0:x1].contiguous() for t in a]
+            out16, noisy_log = dn.torch_reference(torch.from_numpy(p), *crop, spp)
+            ref = torch.clamp(torch.expm1(noisy_log + out16[:, :3]), min=0).permute(0, 2, 3, 1)[0].numpy()
+            m = [0 if y0 == 0 else 96, 384 if y1 == H else 288, 0 if x0 == 0 else 96, 384 if x1 == W else 288]
+            got, want = out[y0:y1, x0:x1][m[0]:m[1], m[2]:m[3]], ref[m[0]:m[1], m[2]:m[3]]
+            err = np.abs(got - want)
+            assert np.allclose(got, want, rtol=2e-2, atol=2e-2), (H, y0, err.max())
+            assert err.mean() < 2e-3
