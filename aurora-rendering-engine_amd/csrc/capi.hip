@@ -31,10 +31,16 @@ constexpr int kTailBlocksPerCu = 5;
 constexpr int kTailWideOneBlocksPerCu = 6;
 constexpr int kTailFlatBlocksPerCu = 8;
 constexpr uint32_t kSortMinNodes = 1u << 21;
-// render bounces by the group walk from this many primitives on (wavefront
-// renders of 5.2 M paths, lane walk -> group walk: 488 spheres 3.1 -> 3.5 ms,
-// 1000 primitives 2.2 -> 2.5, 50 k 7.1 -> 6.4, 190 k 10.4 -> 9.2, 800 k
-// overlapping 10.0 -> 7.4)
+// Render bounces by the group walk where at least half of a call's paths are in
+// scenes of this many primitives or more.  Wavefront renders of 5.2 M paths, lane
+// walk / group walk in ms, scattered scenes and (overlapping ones):
+//   one scene      8 k 4.9/5.4 (6.1/6.5)   16 k 5.9/6.4 (5.5/5.3)   32 k 7.4/7.7 (4.9/4.4)
+//                 64 k 9.3/9.5 (5.7/4.7)  190 k 13.2/12.9 (6.8/5.4)
+//   four scenes    8 k 6.0/6.0 (6.3/6.8)   16 k 7.4/7.1 (5.8/5.9)   32 k 9.2/8.6 (5.4/5.1)
+//                 64 k 11.4/10.5 (6.2/5.3) 190 k 15.8/14.3 (7.2/6.1)
+// With the fused tail from 2^20 live paths on the walks differ by less: the group
+// walk takes 1.12 (1.01) of the lane walk's time at 16 k, 1.06 (1.01) at 32 k, 0.98
+// (0.91) at 190 k for one scene, 1.03 (1.04), 0.98 (1.05), 0.93 (0.98) for four.
 constexpr uint32_t kGroupMinPrims = 16384;
 // The default tree's flat walk: one scene of few leaves whose boxes a ray enters
 // at least one of on average (overlap: flat_build's), where a tree has little to

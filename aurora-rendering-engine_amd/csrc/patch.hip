@@ -572,9 +572,12 @@ Status plan_frame(std::vector<HTri>& scene, const aurora_patch_config& cfg, P3 e
     };
     const size_t work = items.size() * scene.size();
     const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
-    // (the mirror hall of 444 triangles at 1920x1080, 9,482 textures: 2.17 ms with
-    // one thread, 0.80 with four, 0.54 with eight; more gain nothing, for the
-    // largest subtree is then the longest piece and each thread costs its start)
+    // (the mirror hall of 444 triangles at 1920x1080, 9,482 textures: plan 2.17 ms
+    // with one thread, 0.80 with four, 0.54 with eight on eight cores.  On a host
+    // with more, eight and sixteen take 0.81 and 0.73; 4x4, 8x8 and 12x12 equal
+    // mirrors in a tiled room 0.26 and 0.32, 0.40 and 0.38, 0.54 and 0.48: the
+    // starts of more threads cost what they gain on small frames, and each keeps
+    // tables)
     size_t n_threads = work < 8192 ? 1 : std::min<size_t>({kPlanThreads, hw, items.size()});
     if (max_threads) n_threads = std::min<size_t>(n_threads, max_threads);
     // largest projected area first: the big subtrees start early, so the last

@@ -127,7 +127,7 @@ __global__ __launch_bounds__(kBlock) void k_extend(ExtendArgs a) {
     };
 
     WaveClaims claims;
-    claims.init(a.pool, n, 64u, 0u);
+    claims.init(a.pool, n, 64u);
     for (;;) {
         const bool idle = (ri == kNone) && !done;
         const uint64_t im = __ballot(idle);
@@ -297,7 +297,7 @@ __device__ __forceinline__ void group_trace(const IO& io, uint32_t n, uint32_t* 
     group_init(w, sh.g, spill + 2 * (size_t)(blockIdx.x * kGroupBlockRays + (threadIdx.x >> 2)), ray, slot);
     GroupScene sc = io.scene();
     WaveClaims claims;
-    claims.init(pool, n, kGroupRays, 0u);
+    claims.init(pool, n, kGroupRays);
     uint32_t ri = kNone;
     uint32_t head = 0, tail = 0;  // the batch's rays not yet taken
     // the next batch, in registers
@@ -403,7 +403,7 @@ __global__ __launch_bounds__(kBlock) void k_query_lanes(QueryArgs a) {
     v3 o = V(0, 0, 0), d = V(0, 0, 0);
     WideWalk w{};
     WaveClaims claims;
-    claims.init(a.pool, a.n, 64u, 0u);
+    claims.init(a.pool, a.n, 64u);
     for (;;) {
         const bool idle = (ri == kNone) && !done;
         const uint64_t im = __ballot(idle);

@@ -202,8 +202,8 @@ struct WaveClaims {
     uint32_t* pools;
     uint32_t n, ranges, at, lo, hi, count, batch, next, end;  // at: 8 * range + counter
     bool open;
-    // batch_size 0: about an eighth of a wave's share, at least per_wave
-    __device__ __forceinline__ void init(uint32_t* p, uint32_t items, uint32_t per_wave, uint32_t batch_size) {
+    // batches of about an eighth of a wave's share, at least per_wave
+    __device__ __forceinline__ void init(uint32_t* p, uint32_t items, uint32_t per_wave) {
         n = items;
         pools = p;
         next = end = 0u;
@@ -216,7 +216,7 @@ struct WaveClaims {
             end = min(n, next + per_wave);
             return;
         }
-        batch = batch_size ? batch_size : min(4096u, max(per_wave, n / (gridDim.x * waves * 8u) + 1u));
+        batch = min(4096u, max(per_wave, n / (gridDim.x * waves * 8u) + 1u));
         batch = __builtin_amdgcn_readfirstlane(batch);
         at = (blockIdx.x % ranges) * 8u + (blockIdx.x / ranges) % 8u;
         enter();
@@ -242,7 +242,7 @@ struct WaveClaims {
             c = __builtin_amdgcn_readfirstlane(c);
             if (c < count) {
                 next = __builtin_amdgcn_readfirstlane(lo + (8u * c + (at & 7u)) * batch);
-                end = __builtin_amdgcn_readfirstlane(min(hi, next + batch));
+                end = __builtin_amdgcn_readfirstlane(next + min(hi - next, batch));
                 break;
             }
             bool left = false;

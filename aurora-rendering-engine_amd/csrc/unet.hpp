@@ -1,10 +1,19 @@
 // unet.hpp — internal interface of the denoiser: kernel launchers
-// (unet_kernels.hip) and the U-Net that strings them together (unet.hip).
+// (unet_conv.hip, unet_grad.hip, unet_kernels.hip) and the U-Net that strings
+// them together (unet.hip).
 #pragma once
 
 #include "internal.hpp"
 
 namespace aur {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef uint16_t u16;
+
+__device__ __forceinline__ float bf2f(u16 h) { return __uint_as_float((uint32_t)h << 16); }
+// round to nearest even (gfx950's v_cvt_pk_bf16_f32; NaN stays NaN)
+__device__ __forceinline__ u16 f2bf(float f) { return __builtin_bit_cast(u16, (__bf16)f); }
 
 // Convolution input: full-resolution A (Ca channels) concatenated with a
 // half-resolution B (Cb channels) read through nearest upsampling.

@@ -22,12 +22,6 @@
 namespace aur {
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef uint16_t u16;
-
-__device__ __forceinline__ float bf2f(u16 h) { return __uint_as_float((uint32_t)h << 16); }
-__device__ __forceinline__ u16 f2bf(float f) { return __builtin_bit_cast(u16, (__bf16)f); }
 __device__ __forceinline__ uint32_t pack2(float a, float b) { return (uint32_t)f2bf(a) | ((uint32_t)f2bf(b) << 16); }
 
 union Frag {
@@ -351,7 +345,10 @@ Status launch(const ConvArgs& p, int groups, hipStream_t s) {
 // Two rows per wave read a 1.29x halo instead of 1.55x and use every weight
 // fragment eight times; from 512 blocks (two per CU) on: inference 517 us, 519
 // from 256, 542 from 1024, 536 never; a training batch, whose layers have at most
-// 256 such blocks, 790 us, and 830 with the limit at 256.
+// 256 such blocks, 790 us, and 830 with the limit at 256.  The tiles of the layers
+// without a pooled output must also leave room for two blocks per CU.  With one,
+// 64 channels take 95 KB, one block per CU, which still beats a pooling kernel of
+// its own: 2048x2048 1616 us against 1627, 4096x4096 6003 against 6065.
 // Pixel blocks of the one-row-per-wave form below which a layer splits its
 // output channels over the grid (one 16-channel tile per wave), and of the
 // two-row form from which that one is taken.

@@ -10,13 +10,6 @@
 namespace aur {
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef uint16_t u16;
-
-__device__ __forceinline__ float bf2f(u16 h) { return __uint_as_float((uint32_t)h << 16); }
-__device__ __forceinline__ u16 f2bf(float f) { return __builtin_bit_cast(u16, (__bf16)f); }
-
 union Frag {
     uint4 u;
     uint32_t w[4];
@@ -378,8 +371,8 @@ __global__ __launch_bounds__(256) void k_skip_grad(const float* __restrict__ ski
 
 inline unsigned nblocks(size_t n) { return (unsigned)((n + 255) / 256); }
 
-// blocks of a job: a tile or two each, and few enough that the partials stay
-// small against the activations
+// blocks of a job: at most kDwBlocks, so that the partials stay small against the
+// activations (full resolution of an 8 x 128^2 batch: eight tiles each)
 uint32_t job_blocks(const DwPart& p) {
     const uint32_t tiles = (uint32_t)p.N * ((p.H + kRows - 1) / kRows) * ((p.W + kPix - 1) / kPix);
     return std::max(1u, std::min(tiles, kDwBlocks));
@@ -423,10 +416,11 @@ Status weight_grads(const DwPart* parts, int n, float* scratch, hipStream_t s) {
 #define AUR_DW(I, O) \
     case 4 * (I) + (O): k_dw<I, O><<<blocks, 256, lds, s>>>(a); break;
                 switch (4 * nci + nco) {
-                    AUR_DW(1, 1) AUR_DW(1, 2) AUR_DW(1, 3) AUR_DW(1, 4)
-                    AUR_DW(2, 1) AUR_DW(2, 2) AUR_DW(2, 3) AUR_DW(2, 4)
-                    AUR_DW(3, 1) AUR_DW(3, 2) AUR_DW(3, 3) AUR_DW(3, 4)
-                    AUR_DW(4, 1) AUR_DW(4, 2) AUR_DW(4, 3) AUR_DW(4, 4)
+                    AUR_DW(1, 2)
+                    AUR_DW(2, 1) AUR_DW(2, 2) AUR_DW(2, 3)
+                    AUR_DW(3, 2) AUR_DW(3, 3) AUR_DW(3, 4)
+                    AUR_DW(4, 3) AUR_DW(4, 4)
+                    default: return Status{AURORA_ERR_INVALID, "denoiser: no weight gradient for these channel counts"};
                 }
 #undef AUR_DW
                 AUR_HIP(hipGetLastError());

@@ -11,14 +11,6 @@
 namespace aur {
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef uint16_t u16;
-
-__device__ __forceinline__ float bf2f(u16 h) { return __uint_as_float((uint32_t)h << 16); }
-// round to nearest even (gfx950's v_cvt_pk_bf16_f32; NaN stays NaN)
-__device__ __forceinline__ u16 f2bf(float f) { return __builtin_bit_cast(u16, (__bf16)f); }
-
 union Pack8 {
     uint4 u;
     bf16x8 v;
