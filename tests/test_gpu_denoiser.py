@@ -38,13 +38,14 @@ def random_params(n, seed):
     return (rng.normal(size=n) * 0.05).astype(np.float32)
 
 
-# Launch shapes (conv3x3_forward picks them from the pixel-block count of
-# each layer).  32x48: every layer has fewer than 128 blocks, so every conv
+# Launch shapes (unet_conv.hip's dispatch picks them from the pixel-block count
+# of each layer).  32x48: every layer has fewer than 128 blocks, so every conv
 # takes the channel-split form (one 16-channel tile per wave, NT = 1).
-# 1024x1024, the inference workload: levels 0-2 take the wide waves with
-# NT = 2, 3, 4 (32, 48, 64 output channels; 4096, 1024, 256 blocks), rows of
-# 16 and 4 segments of 64 pixels with their halos, encoder and concatenating
-# decoder forms; level 3 (128^2, 64 blocks) the channel split.
+# 1024x1024, the inference workload: levels 0 and 1 take two rows per wave where
+# their tiles fit 80 KB (32 and 48 output channels, NT = 2 and 3, pooling in the
+# epilogue; 2048 and 512 blocks), level 2 one row per wave (64 channels, NT = 4,
+# 256 blocks), rows of 16 to 4 segments of 64 pixels with their halos, encoder and
+# concatenating decoder forms; level 3 (128^2, 64 blocks) the channel split.
 @pytest.mark.parametrize("H,W", [(32, 48), (1024, 1024)])
 def test_forward_matches_torch(ctx, H, W):
     print("denoiser forward", H, W, flush=True)
@@ -63,9 +64,9 @@ def test_forward_matches_torch(ctx, H, W):
 
 
 # 8 x 128^2 is the training step's batch: the forward and the data-gradient
-# convolutions take NT = 2 (level 0, 512 blocks) and NT = 3 (level 1, 128
-# blocks) and two row segments per 128-pixel row; levels 2-3 the channel
-# split; the weight gradient reduces 1024 partial blocks per tile.
+# convolutions take one row per wave, NT = 2 (level 0, 512 blocks) and NT = 3
+# (level 1, 128 blocks), and two row segments per 128-pixel row; levels 2-3 the
+# channel split; the weight gradient sums up to 128 partial blocks per input part.
 @pytest.mark.parametrize("B,H,W", [(2, 16, 32), (8, 128, 128)])
 @pytest.mark.parametrize("kind", ["log", "rel"])
 def test_gradients_match_torch_autograd(ctx, kind, B, H, W):
